@@ -114,6 +114,15 @@ __device__ __forceinline__ int64_t snap1(double v, double s, double t, int64_t v
     return vv == vmax ? vv - 1 : vv;
 }
 
+// For a segment with both ends in [lo, hi], starting at v0 with the delta d its column's
+// precision gives: whether _clipt leaves it whole.  Its q are then >= 0, so only the
+// `p > 0 and q < p` branch could act, for (p, q) = (-d, v0 - lo) and (d, hi - v0).  (The
+// exact q is never less than the exact delta, but a float32 delta that rounds away from
+// zero can exceed it when a vertex lies on a bound.)
+__device__ __forceinline__ bool unclipped(double v0, double d, double lo, double hi) {
+    return __dsub_rn(v0, lo) >= -d && __dsub_rn(hi, v0) >= d;
+}
+
 // draw_segment, line.py:1045-1095, for coordinates of column types TX / TY.
 template <typename TX, typename TY, typename I, typename S>
 __device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bool segment_start,
@@ -127,16 +136,11 @@ __device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bo
     double t0 = 0.0, t1 = 1.0;
     const double dx1 = (double)(TX)(x1c - x0c);  // column precision (numba typing)
     const double dy1 = (double)(TY)(y1c - y0c);
-    // Both ends inside the view and each delta equal to the float64 difference of its
-    // ends: then every _clipt call leaves (t0, t1) = (0, 1) and they are skipped.  (With
-    // x1 <= xmax, the exact xmax - x0 is >= the exact x1 - x0, so the rounded q = xmax - x0
-    // is >= p = fl64(x1 - x0); _clipt's q < p branch cannot fire, and likewise for the
-    // other three bounds.)  A float32 delta that rounds away from the float64 one can
-    // exceed q when a vertex lies on a bound; _clipt then clips (t1 < 1), so such a
-    // segment takes the four calls.
+    // Both ends inside the view and no _clipt call able to shorten the segment: (t0, t1)
+    // stays (0, 1) and the four calls, with their divisions, are skipped.
     const bool inside = a.xmin <= x0 && x0 <= a.xmax && a.xmin <= x1 && x1 <= a.xmax &&
                         a.ymin <= y0 && y0 <= a.ymax && a.ymin <= y1 && y1 <= a.ymax &&
-                        dx1 == __dsub_rn(x1, x0) && dy1 == __dsub_rn(y1, y0);
+                        unclipped(x0, dx1, a.xmin, a.xmax) && unclipped(y0, dy1, a.ymin, a.ymax);
     if (!inside) {
         if (!clipt(-dx1, __dsub_rn(x0, a.xmin), t0, t1)) skip = true;
         if (!clipt(dx1, __dsub_rn(a.xmax, x0), t0, t1)) skip = true;
@@ -200,156 +204,305 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a, Planes p) {
     }
 }
 
+// ---- count only: rasterising into LDS ------------------------------------------------
+// The lines of a count (no value column, no categorizer) are drawn into a box of the
+// canvas held in LDS, and the box's non-zero cells are added to the count plane with one
+// global atomic each; a pixel outside the box goes straight to the global plane, so the
+// result never depends on the box.  Random LDS u32 atomics run at 5.1 T/s here, global
+// ones at 14-27 G/s.
+constexpr int kBoxThreads = 1024;
+constexpr int kBoxLds = 160 * 1024 - 1024;  // the box, less 1 KB for the kernels' own words
+
+// The box's counters in the workgroup's dynamic LDS.
+extern __shared__ uint32_t box_cells[];
+
+using lds_u32 = __attribute__((address_space(3))) uint32_t;
+
+// Count one pixel at an LDS address (32-bit, from Box::at): an address the walk steps
+// itself, so that no base is added to it again for every pixel.
+__device__ __forceinline__ void box_add(uint32_t addr) {
+    __hip_atomic_fetch_add((lds_u32 *)(uintptr_t)addr, 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Columns [c0, c0 + cols) and rows [r0, r0 + rows) of the canvas; odd row pitch, so that a
+// column's cells spread over the LDS banks.
+struct Box {
+    int32_t c0, r0, cols, rows, pitch;
+    __device__ __forceinline__ bool has(int32_t x, int32_t y) const {
+        return (uint32_t)(x - c0) < (uint32_t)cols && (uint32_t)(y - r0) < (uint32_t)rows;
+    }
+    __device__ __forceinline__ uint32_t at(int32_t x, int32_t y) const {
+        return (uint32_t)(uintptr_t)(lds_u32 *)box_cells + (uint32_t)((y - r0) * pitch + (x - c0)) * 4u;
+    }
+};
+
+// _bresenham for an unclipped segment whose ends (so all its pixels) lie in the box.  With
+// n steps along the major axis and m <= n along the minor one, the reference's error term
+// has moved the minor axis floor((2 m i + n - b) / 2 n) times after i steps, b = 1 where
+// the major axis runs backwards (its tie rule), else 0.  Short segments hold that quotient,
+// moved up by 1 / 4n -- half of its distance to the next value above --, in fixed point with
+// 20 fractional bits: n steps of a slope that is off by less than 1.5 * 2^-20 stay within
+// 1 / 4n for n < kDdaMax, so the floor is exact.  A step is then an add, a shift, a
+// multiply-add and an add, with no compare or select.  Long ones keep the error term (its
+// half, less b, so that the reference's `err >= 0 && (err || i > 0)` is err >= 0).
+// common: a number of steps that every active lane takes (uniform), so that those run
+// without a lane mask.
+constexpr int32_t kDdaMax = 256;
+
+__device__ __forceinline__ void box_walk(uint32_t at, int32_t dx, int32_t dy, uint32_t pitch4,
+                                         bool start, int32_t common) {
+    const int32_t ax = dx < 0 ? -dx : dx, ay = dy < 0 ? -dy : dy;
+    const bool xm = ax >= ay;
+    const int32_t n = xm ? ax : ay, m = xm ? ay : ax;
+    if (start || n == 0) box_add(at);
+    const int32_t ox = dx < 0 ? -4 : 4, oy = dy < 0 ? -(int32_t)pitch4 : (int32_t)pitch4;
+    const int32_t o1 = xm ? ox : oy, o2 = xm ? oy : ox;  // along the major axis; the minor
+    const bool fwd = (xm ? dx : dy) > 0;
+    if (n < kDdaMax) {
+        const float rn = __builtin_amdgcn_rcpf((float)n);
+        const uint32_t slope = (uint32_t)((float)m * rn * 1048576.0f);
+        const int32_t quarter = (int32_t)(rn * 262144.0f);
+        uint32_t acc = 524288u + (uint32_t)(fwd ? quarter : -quarter);
+        int32_t i = 0;
+        auto step = [&]() {
+            acc += slope;
+            at += (uint32_t)o1;
+            box_add((uint32_t)(__mul24((int32_t)(acc >> 20), o2) + (int32_t)at));
+        };
+#pragma unroll 4
+        for (; i < common; ++i) step();
+        uint32_t left = (uint32_t)(n - i);
+        while (!__builtin_sub_overflow(left, 1u, &left)) step();
+        return;
+    }
+    const int32_t e1 = 2 * m, e2 = 2 * (m - n);
+    int32_t err = e1 - n - (fwd ? 0 : 1);
+    for (int32_t i = n; i > 0; --i) {
+        const bool both = err >= 0;
+        at += (uint32_t)(both ? o1 + o2 : o1);
+        err += both ? e2 : e1;
+        box_add(at);
+    }
+}
+
+struct BoxSink {
+    uint32_t *count;
+    int32_t W, H;
+    Box box;
+    __device__ __forceinline__ void operator()(int32_t x, int32_t y) const {
+        if (x < 0) x += W;  // numba's negative-index wraparound
+        if (y < 0) y += H;
+        if ((uint32_t)x >= (uint32_t)W || (uint32_t)y >= (uint32_t)H) return;
+        if (box.has(x, y)) box_add(box.at(x, y));
+        else atomicAdd(count + (int64_t)y * W + x, 1u);
+    }
+    template <typename I>
+    __device__ __forceinline__ void walk(bool start, I x0, I x1, I y0, I y1, bool clipped) const {
+        bresenham<I>(*this, start, x0, x1, y0, y1, clipped);
+    }
+};
+
+// Pixel of a coordinate (snap1 in 32 bits); a value far off the canvas (a degenerate view)
+// or NaN saturates, so it is in no box.  vmax: snap_max of the axis's last pixel.
+template <bool LOG>
+__device__ __forceinline__ int32_t snap_in(double v, double s, double t, int32_t vmax, int32_t log) {
+    const double d = __dadd_rn(__dmul_rn(LOG ? axis_map(v, log) : v, s), t);
+    int32_t p;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(p) : "v"(d));  // truncates and saturates
+    return p == vmax ? p - 1 : p;
+}
+__device__ __forceinline__ int32_t snap_max(int64_t vmax) {  // (no pixel is the lowest integer)
+    return vmax == (int64_t)(int32_t)vmax ? (int32_t)vmax : INT32_MIN;
+}
+
+__device__ __forceinline__ void box_flush(const Box &b, uint32_t *count, int32_t W, int32_t H) {
+    for (int i = threadIdx.x; i < b.rows * b.pitch; i += kBoxThreads) {
+        const uint32_t v = box_cells[i];
+        if (!v) continue;
+        const int32_t r = i / b.pitch, c = i - r * b.pitch;
+        const int32_t x = b.c0 + c, y = b.r0 + r;
+        if (c < b.cols && x < W && y < H) atomicAdd(count + (int64_t)y * W + x, v);
+    }
+}
+
 // ---- x-constant series, count only: LDS strips ---------------------------------------
 // Lines of an axis-1 frame whose x is shared (x_line_stride == 0, LinesAxis1XConstant,
 // line.py:334-380) put segment j of every line between the same two x values, so the
 // pixels of segments [j0, j0 + k) of all lines fall in one narrow band of columns.
 // Workgroup (s, b) rasterises segments [s*k, s*k + k) of lines [b*L, b*L + L) into an
-// LDS copy of that band (all H rows, row pitch odd so that rows spread over the LDS
-// banks), then adds the band's non-zero cells to the count plane with one global atomic
-// per cell.  A pixel outside the band (x not monotone, wraparound) goes straight to the
-// global plane, so the result never depends on the band guess.
-constexpr int kStripThreads = 1024;
-constexpr int kStripLds = 160 * 1024;
+// LDS copy of that band (all H rows).
+//
+// Bound by instruction issue (2.3 G pixel updates of 1M x 256 series: 0.45 ms of LDS
+// atomics, 1.03 GB of columns: 0.2 ms).  So what all lines share -- the snapped x of each
+// vertex, whether it is in the view -- is worked out once per workgroup, each vertex's y is
+// projected once (not once per segment it ends), in 32 bits, and only segments that
+// clipping could shorten take draw_segment: telling those by an inexact float32 delta sent
+// a lane of nearly every wave there (values near zero), 2.21 against 1.54 ms.  The
+// fixed-point walk, its common steps without a lane mask: 1.54 -> 1.10 ms.  Before all of
+// it 2.89 ms (2048 x 1024).
 constexpr int kStripMaxK = 8;        // segments per strip
 
-// The band, [H][pitch] counters in the workgroup's dynamic LDS.  Named at file scope so
-// that every access through the sink below compiles to an LDS (ds_*) atomic.
-extern __shared__ uint32_t strip_band[];
+struct StripSeg {
+    int32_t px0, px1;  // snapped ends
+    int32_t flags;     // SEG_* bits
+    int32_t pad;
+    double x0, x1;
+};
+enum : int32_t {
+    SEG_FAST = 1,   // both ends in the view and in the band's columns, unclipped in x
+    SEG_SKIP = 2,   // nothing of it can be drawn (an end missing, or both outside)
+    SEG_START = 4   // the x before it is missing
+};
 
-struct StripSink {
-    uint32_t *count;
-    int32_t W, H, c0, cols, pitch;
-    __device__ __forceinline__ void operator()(int32_t x, int32_t y) const {
-        if (x < 0) x += W;  // numba's negative-index wraparound
-        if (y < 0) y += H;
-        if ((uint32_t)x >= (uint32_t)W || (uint32_t)y >= (uint32_t)H) return;
-        const uint32_t cx = (uint32_t)(x - c0);
-        if (cx < (uint32_t)cols) atomicAdd(&strip_band[y * pitch + cx], 1u);
-        else atomicAdd(count + (int64_t)y * W + x, 1u);
-    }
-    // The pixels of a walk lie in the box of its ends.  When that box is inside the band
-    // and the canvas, the walk runs without per-pixel checks as one loop over the major
-    // axis (the two loops of _bresenham with the axes named by role: same pixels, same
-    // tie rule); otherwise it is the checked walk.
-    template <typename I>
-    __device__ __forceinline__ void walk(bool start, I x0, I x1, I y0, I y1, bool clipped) const {
-        const I xl = x0 < x1 ? x0 : x1, xh = x0 < x1 ? x1 : x0;
-        const I yl = y0 < y1 ? y0 : y1, yh = y0 < y1 ? y1 : y0;
-        if (!(xl >= c0 && xh < c0 + cols && xh < W && yl >= 0 && yh < H)) {
-            bresenham<I>(*this, start, x0, x1, y0, y1, clipped);
-            return;
-        }
-        uint32_t *base = strip_band - c0;  // band cell of pixel (x, y): base[y * pitch + x]
-        I dx = x1 - x0;
-        const I ix = (dx > 0) - (dx < 0);
-        dx = (dx < 0 ? -dx : dx) * 2;
-        I dy = y1 - y0;
-        const I iy = (dy > 0) - (dy < 0);
-        dy = (dy < 0 ? -dy : dy) * 2;
-        if (!clipped && !(dx | dy)) {
-            atomicAdd(&base[y0 * pitch + x0], 1u);
-            return;
-        }
-        if (start) atomicAdd(&base[y0 * pitch + x0], 1u);
-        const bool xmajor = dx >= dy;
-        I a = xmajor ? x0 : y0, a1 = xmajor ? x1 : y1, b = xmajor ? y0 : x0;
-        const I ia = xmajor ? ix : iy, ib = xmajor ? iy : ix;
-        const I da = xmajor ? dx : dy, db = xmajor ? dy : dx;
-        // LDS offsets of one step along each axis
-        const I sa = xmajor ? ia : ia * pitch, sb = xmajor ? ib * pitch : ib;
-        I off = y0 * pitch + x0;
-        I err = 2 * db - da;
-        while (a != a1) {
-            if (err >= 0 && (err || ia > 0)) {
-                err -= 2 * da;
-                b += ib;
-                off += sb;
-            }
-            err += 2 * db;
-            a += ia;
-            off += sa;
-            atomicAdd(&base[off], 1u);
-        }
-        (void)b;
+// Line l's samples j0 .. j0 + K (the last one repeated past nv), and whether sample j0 - 1
+// is missing.
+template <typename TY, int K>
+struct StripRow {
+    TY y[K + 1];
+    TY prev;
+    __device__ __forceinline__ void load(const LineArgs &a, int64_t j0, int nv, int64_t l) {
+        const TY *Y = reinterpret_cast<const TY *>(a.y) + l * a.yls;
+#pragma unroll
+        for (int q = 0; q <= K; ++q) y[q] = Y[(j0 + (q < nv ? q : nv - 1)) * a.yvs];
+        prev = Y[(j0 > 0 ? j0 - 1 : 0) * a.yvs];
     }
 };
 
-template <typename TX, typename TY>
-__global__ __launch_bounds__(kStripThreads) void lines_xconst_strip_kernel(LineArgs a,
-                                                                           uint32_t *count,
-                                                                           int32_t k,
-                                                                           int32_t cols,
-                                                                           int32_t pitch,
-                                                                           int64_t lpb) {
-    uint32_t *band = strip_band;
-    __shared__ int32_t s_c0;
+template <typename TX, typename TY, int K, bool LOG>
+__global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArgs a,
+                                                                         uint32_t *count,
+                                                                         int32_t k,
+                                                                         int32_t pitch,
+                                                                         int64_t lpb) {
+    // (after the band in dynamic LDS: with no static LDS the band starts at address 0)
+    StripSeg *s_seg = reinterpret_cast<StripSeg *>(box_cells + ((a.H * pitch + 3) & ~3));
     const TX *X = reinterpret_cast<const TX *>(a.x);
-    const TY *Y = reinterpret_cast<const TY *>(a.y);
     const int64_t nseg = a.nverts - 1;
     const int64_t j0 = (int64_t)blockIdx.x * k;
     const int64_t j1 = j0 + k < nseg ? j0 + k : nseg;  // segments [j0, j1)
+    const int ns = (int)(j1 - j0), nv = ns + 1;
     const int64_t l0 = (int64_t)blockIdx.y * lpb;
     const int64_t l1 = l0 + lpb < a.nlines ? l0 + lpb : a.nlines;
-    if (threadIdx.x == 0) {
-        // first column of the band: the leftmost snapped vertex of the strip, with x
-        // clamped to the view as clipping would (a clipped end lies between its vertices)
-        int64_t lo = a.W;
-        for (int64_t j = j0; j <= j1; ++j) {
-            double x = (double)X[j * a.xvs];
-            if (x != x) continue;
-            x = x < a.xmin ? a.xmin : (x > a.xmax ? a.xmax : x);
-            const int64_t c = snap1(x, a.sx, a.tx, a.xxmax, a.xlog);
-            lo = c < lo ? c : lo;
-        }
-        s_c0 = (int32_t)(lo < 0 ? 0 : (lo > a.W ? a.W : lo));
+    const int tid = threadIdx.x;
+    // first column of the band: the leftmost snapped vertex of the strip, with x clamped
+    // to the view as clipping would (a clipped end lies between its vertices)
+    int64_t lo = a.W;
+    for (int64_t j = j0; j <= j1; ++j) {
+        double x = (double)X[j * a.xvs];
+        if (x != x) continue;
+        x = x < a.xmin ? a.xmin : (x > a.xmax ? a.xmax : x);
+        const int64_t c = snap1(x, a.sx, a.tx, a.xxmax, a.xlog);
+        lo = c < lo ? c : lo;
     }
-    for (int i = threadIdx.x; i < a.H * pitch; i += kStripThreads) band[i] = 0u;
-    __syncthreads();
-    StripSink put;
+    BoxSink put;
     put.count = count; put.W = a.W; put.H = a.H;
-    put.c0 = s_c0; put.cols = cols; put.pitch = pitch;
-    const int nv = (int)(j1 - j0) + 1;  // vertices j0 .. j1
-    TX xs[kStripMaxK + 1];
-#pragma unroll
-    for (int q = 0; q <= kStripMaxK; ++q) xs[q] = q < nv ? X[(j0 + q) * a.xvs] : TX(0);
-    const bool xprev_nan = j0 > 0 && X[(j0 - 1) * a.xvs] != X[(j0 - 1) * a.xvs];
-    for (int64_t l = l0 + threadIdx.x; l < l1; l += kStripThreads) {
-        const TY *Yl = Y + l * a.yls;
-        TY ys[kStripMaxK + 1];
-#pragma unroll
-        for (int q = 0; q <= kStripMaxK; ++q) ys[q] = q < nv ? Yl[(j0 + q) * a.yvs] : TY(0);
-        // segment_start (line.py:1371-1373): the first segment of a line, or one whose
-        // previous vertex is missing
-        bool start = true;
-        if (j0 > 0) {
-            const TY yp = Yl[(j0 - 1) * a.yvs];
-            start = xprev_nan || (yp != yp);
+    put.box.c0 = __builtin_amdgcn_readfirstlane((int32_t)(lo < 0 ? 0 : (lo > a.W ? a.W : lo)));
+    put.box.r0 = 0;
+    put.box.cols = pitch; put.box.rows = a.H; put.box.pitch = pitch;
+    for (int i = tid; i < a.H * pitch; i += kBoxThreads) box_cells[i] = 0u;
+    const int32_t xxmax = snap_max(a.xxmax), yymax = snap_max(a.yymax);
+    if (tid <= ns) {  // (one past the last: read ahead, never drawn)
+        const int64_t j = j0 + (tid < ns ? tid : ns - 1);
+        const TX x0c = X[j * a.xvs], x1c = X[(j + 1) * a.xvs];
+        const double x0 = (double)x0c, x1 = (double)x1c;
+        StripSeg g;
+        g.x0 = x0; g.x1 = x1; g.pad = 0; g.flags = 0;
+        g.px0 = snap_in<LOG>(x0, a.sx, a.tx, xxmax, a.xlog);
+        g.px1 = snap_in<LOG>(x1, a.sx, a.tx, xxmax, a.xlog);
+        const auto col = [&](int32_t c) {
+            return c >= 0 && c < a.W && (uint32_t)(c - put.box.c0) < (uint32_t)pitch;
+        };
+        if (a.xmin <= x0 && x0 <= a.xmax && a.xmin <= x1 && x1 <= a.xmax && col(g.px0) &&
+            col(g.px1) && unclipped(x0, (double)(TX)(x1c - x0c), a.xmin, a.xmax))
+            g.flags |= SEG_FAST;
+        if (x0 != x0 || x1 != x1 || (x0 < a.xmin && x1 < a.xmin) || (x0 > a.xmax && x1 > a.xmax))
+            g.flags |= SEG_SKIP;
+        if (j > 0) {
+            const TX xp = X[(j - 1) * a.xvs];
+            if (xp != xp) g.flags |= SEG_START;
         }
-        // segments drawn from the front of shifting register windows (a rolled loop with
-        // constant register indices: one copy of the rasteriser, no indexed registers)
-        TX xq[kStripMaxK + 1];
-#pragma unroll
-        for (int q = 0; q <= kStripMaxK; ++q) xq[q] = xs[q];
-#pragma unroll 1
-        for (int q = 0; q + 1 < nv; ++q) {
-            draw_segment<TX, TY, int32_t>(a, put, start, xq[0], xq[1], ys[0], ys[1]);
-            start = (xq[0] != xq[0]) || (ys[0] != ys[0]);
-#pragma unroll
-            for (int i = 0; i < kStripMaxK; ++i) {
-                xq[i] = xq[i + 1];
-                ys[i] = ys[i + 1];
-            }
-        }
+        s_seg[tid] = g;
     }
     __syncthreads();
-    const int32_t c0 = s_c0;
-    for (int i = threadIdx.x; i < a.H * pitch; i += kStripThreads) {
-        const uint32_t v = band[i];
-        if (!v) continue;
-        const int32_t y = i / pitch, cx = i - y * pitch;
-        if (cx < cols && c0 + cx < a.W) atomicAdd(count + (int64_t)y * a.W + c0 + cx, v);
+    const uint32_t pitch4 = (uint32_t)pitch * 4u;
+    // the next line's samples are loaded while this line is drawn
+    StripRow<TY, K> row, far;
+    const int64_t lt = l0 + tid;
+    if (lt < l1) row.load(a, j0, nv, lt);
+    for (int64_t l = lt; l < l1; l += kBoxThreads) {
+        far.load(a, j0, nv, l + kBoxThreads < l1 ? l + kBoxThreads : l);
+        // one vertex per step: its place in the view and its pixel row, once
+        bool gap = j0 == 0 || row.prev != row.prev;  // the sample before is missing
+        double y0 = (double)row.y[0];
+        bool in0 = a.ymin <= y0 && y0 <= a.ymax;
+        int32_t py0 = snap_in<LOG>(y0, a.sy, a.ty, yymax, a.ylog);
+        int4 g = *reinterpret_cast<const int4 *>(&s_seg[0]);  // px0, px1, flags
+        // segments drawn from the front of a shifting register window (a rolled loop with
+        // constant register indices: one copy of the rasteriser, no indexed registers)
+#pragma unroll 1
+        for (int q = 0; q < ns; ++q) {
+            const int32_t px0 = __builtin_amdgcn_readfirstlane(g.x);
+            const int32_t px1 = __builtin_amdgcn_readfirstlane(g.y);
+            const int32_t flags = __builtin_amdgcn_readfirstlane(g.z);
+            g = *reinterpret_cast<const int4 *>(&s_seg[q + 1]);
+            const TY y0c = row.y[0], y1c = row.y[1];
+            const double y1 = (double)y1c;
+            const bool in1 = a.ymin <= y1 && y1 <= a.ymax;
+            const int32_t py1 = snap_in<LOG>(y1, a.sy, a.ty, yymax, a.ylog);
+            const bool start = gap || (flags & SEG_START) != 0;
+            const bool fast = in0 & in1 & ((uint32_t)py0 < (uint32_t)a.H) &
+                              ((uint32_t)py1 < (uint32_t)a.H) &
+                              unclipped(y0, (double)(TY)(y1c - y0c), a.ymin, a.ymax) &
+                              ((flags & SEG_FAST) != 0);
+            const int32_t dx = px1 - px0;
+            if (fast) {
+                box_walk(put.box.at(px0, py0), dx, py1 - py0, pitch4, start, dx < 0 ? -dx : dx);
+            } else if (!(flags & SEG_SKIP)) {
+                // (both ends beyond one bound, or one missing: nothing is drawn)
+                const bool none = y0 != y0 || y1 != y1 || (y0 < a.ymin && y1 < a.ymin) ||
+                                  (y0 > a.ymax && y1 > a.ymax);
+                if (!none)
+                    draw_segment<TX, TY, int32_t>(a, put, start, (TX)s_seg[q].x0, (TX)s_seg[q].x1,
+                                                  y0c, y1c);
+            }
+            gap = y0 != y0;
+            y0 = y1;
+            in0 = in1;
+            py0 = py1;
+#pragma unroll
+            for (int i = 0; i < K; ++i) row.y[i] = row.y[i + 1];
+        }
+        row = far;
     }
+    __syncthreads();
+    box_flush(put.box, count, a.W, a.H);
+}
+
+static int cu_count() {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        int c = 0;
+        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
+            cus = c;
+    }
+    return cus;
+}
+
+template <typename TX, typename TY>
+static int launch_strips(const LineArgs &a, uint32_t *count, int64_t nstrips, int64_t nblocks,
+                         int64_t k, int64_t pitch, int64_t lpb, hipStream_t s) {
+    const size_t lds = (size_t)4 * ((a.H * pitch + 3) & ~3) + sizeof(StripSeg) * (kStripMaxK + 1);
+    // (two band sizes, so that few registers hold samples a strip does not have)
+    auto kern = k <= 4 ? lines_xconst_strip_kernel<TX, TY, 4, false>
+                       : lines_xconst_strip_kernel<TX, TY, kStripMaxK, false>;
+    if (a.xlog || a.ylog) kern = lines_xconst_strip_kernel<TX, TY, kStripMaxK, true>;
+    const hipError_t e = hipFuncSetAttribute((const void *)kern,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
+    hipLaunchKernelGGL(kern, dim3((unsigned)nstrips, (unsigned)nblocks), dim3(kBoxThreads), lds, s, a,
+                       count, (int32_t)k, (int32_t)pitch, lpb);
+    return launch_status();
 }
 
 template <typename TX, typename TY>
@@ -398,38 +551,24 @@ extern "C" int dsx_lines_agg(const dsx_lines_desc *d, const dsx_view *v, const d
     hipStream_t s = as_stream(stream);
     const bool x32 = d->x_dtype == DSX_F32, y32 = d->y_dtype == DSX_F32;
     // x-constant series with count / any only: LDS strips
-    int64_t pitch = kStripLds / (4 * (int64_t)v->height);
+    int64_t pitch = kBoxLds / (4 * (int64_t)v->height);
     if (pitch % 2 == 0) --pitch;
-    if (d->axis == 1 && d->x_line_stride == 0 && !d->val && d->cat.kind == DSX_CAT_NONE &&
-        acc->count && !needs_val && pitch >= 5) {
+    const bool counts = !d->val && d->cat.kind == DSX_CAT_NONE && acc->count && !needs_val;
+    if (counts && d->axis == 1 && d->x_line_stride == 0 && pitch >= 5) {
         const int64_t nseg = d->nverts - 1;
         int64_t k = (pitch - 2) * nseg / v->width;  // segments whose band fits, for x spread evenly
         k = k < 1 ? 1 : (k > kStripMaxK ? kStripMaxK : k);
         const int64_t nstrips = (nseg + k - 1) / k;
-        int dev = 0, cus = 256;
-        if (hipGetDevice(&dev) == hipSuccess) {
-            int c = 0;
-            if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-                c > 0)
-                cus = c;
-        }
+        const int cus = cu_count();
         int64_t nblocks = (cus + nstrips - 1) / nstrips;
         if (nblocks > d->nlines) nblocks = d->nlines;
         if (nblocks < 1) nblocks = 1;
         if (nstrips <= 65535 && nblocks <= 65535) {
             const int64_t lpb = (d->nlines + nblocks - 1) / nblocks;
-            const size_t lds = (size_t)4 * v->height * pitch;
-            auto kern = lines_xconst_strip_kernel<float, float>;
-            if (!x32 && y32) kern = lines_xconst_strip_kernel<double, float>;
-            else if (x32 && !y32) kern = lines_xconst_strip_kernel<float, double>;
-            else if (!x32 && !y32) kern = lines_xconst_strip_kernel<double, double>;
-            const hipError_t e = hipFuncSetAttribute((const void *)kern,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     (int)lds);
-            if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-            hipLaunchKernelGGL(kern, dim3((unsigned)nstrips, (unsigned)nblocks), dim3(kStripThreads),
-                               lds, s, a, p.count, (int32_t)k, (int32_t)pitch, (int32_t)pitch, lpb);
-            return launch_status();
+            return x32 ? (y32 ? launch_strips<float, float>(a, p.count, nstrips, nblocks, k, pitch, lpb, s)
+                              : launch_strips<float, double>(a, p.count, nstrips, nblocks, k, pitch, lpb, s))
+                       : (y32 ? launch_strips<double, float>(a, p.count, nstrips, nblocks, k, pitch, lpb, s)
+                              : launch_strips<double, double>(a, p.count, nstrips, nblocks, k, pitch, lpb, s));
         }
     }
     const int block = 256;
