@@ -406,89 +406,130 @@ struct ScanArgs {
     const double *mean;              // squared-deviation mode (m2 pass)
 };
 
-// How the scan reads a row's category: no categorizer, a one-byte code column (int8 /
-// uint8), or any other categorizer column.
-// CK_CODE8: a one-byte code column read by category codes (no modulo / binning).
-enum : int { CK_NONE = 0, CK_BYTE = 1, CK_ANY = 2, CK_CODE8 = 3 };
+// How a scan reads a row's category: no categorizer, any categorizer column, or one-byte
+// category codes (int8 / uint8, no modulo / binning).
+enum : int { CK_NONE = 0, CK_ANY = 2, CK_CODE8 = 3 };
 
-// Rows of chunk ck handled by this thread.  Every load is issued unconditionally (a row
-// past the end reads the last row and is dropped when binned), so the loads of a chunk
-// are a fixed-length run and the compiler waits for exactly the chunk it bins while the
-// chunks prefetched behind it stay in flight.  Loaded values are not touched here.
-// WIDE (float32 columns, 16-byte aligned, n a multiple of 4 -- checked on the host): the
-// thread's rows are b + 4 tid .. b + 4 tid + 3, one 16-byte load per column (the streams
-// then run ~10 % faster than with a 4-byte load per row: 6.95 against 6.24 TB/s for three
-// columns on one MI355X).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+static int cat_kind(const Cat &c) {
+    if (c.kind == DSX_CAT_NONE) return CK_NONE;
+    return (c.dtype == DSX_I8 || c.dtype == DSX_U8) && c.kind == DSX_CAT_CODES ? CK_CODE8 : CK_ANY;
+}
 
-template <typename TC, typename TV, bool HAS_VAL, int CK, bool WIDE = false>
+// The rows of a chunk a thread bins, in groups of consecutive rows that one wide load a
+// column reads: a group of four where every column is 4 bytes wide (16-byte loads), two
+// groups of two where one has 8 (16 bytes, or 8 of a float32 column), so that the lanes'
+// loads lie side by side.  A load needs 4-byte alignment (a code load none), so any column
+// address and any row count will do: three float32 columns stream at 6.95 TB/s so, 6.24
+// with a 4-byte load a row.  A group that would pass the end reads the table's last rows
+// instead; its rows before `shift` are then not its own.  Tables have at least four rows
+// (pad_rows).  Every load is issued unconditionally and no loaded value is touched here, so
+// that the compiler waits for exactly the chunk it bins while the chunks prefetched behind
+// it stay in flight (a branch around the loads drains them).
+template <typename T, int PER> struct LoadVec;
+template <> struct LoadVec<float, 4> { typedef float T __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct LoadVec<float, 2> { typedef float T __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct LoadVec<double, 2> { typedef double T __attribute__((ext_vector_type(2), aligned(8))); };
+template <int PER> struct LoadCodes { typedef uint32_t T __attribute__((aligned(1))); };
+template <> struct LoadCodes<2> { typedef uint16_t T __attribute__((aligned(1))); };
+
+template <typename TC, typename TV, bool HAS_VAL, int CK>
 struct Rows {
+    static constexpr int kPer = sizeof(TC) == 8 || (HAS_VAL && sizeof(TV) == 8) ? 2 : 4;
+    static constexpr int kGroups = kItems / kPer;
     TC x[kItems], y[kItems];
     TV v[kItems];
-    int64_t c[kItems];
+    uint32_t c8[kGroups];  // CK_CODE8: the groups' one-byte codes
+    int64_t c[kItems];     // CK_ANY: the raw categorizer inputs
+    int32_t shift[kGroups];
 
     __device__ __forceinline__ void load(const PointArgs &a, int64_t ck, int tid) {
-        if constexpr (WIDE) {
-            static_assert(sizeof(TC) == 4 && (!HAS_VAL || sizeof(TV) == 4) &&
-                          (CK == CK_NONE || CK == CK_CODE8) && kItems == 4,
-                          "wide rows: float32 columns (one-byte codes), four rows a thread");
-            int64_t b = ck * kChunk;
-            uint32_t lastq;  // the last readable group of four rows
-            if (b >= a.n) {  // a prefetch past the end: re-read the last four rows
-                b = a.n - 4;
-                lastq = 0;
+        const int64_t b = ck * kChunk;
+        const int64_t end = a.n - kPer;               // the last readable group
+        const int64_t bb = b < end ? b : end;         // uniform
+        const int64_t room = end - bb, past = b - bb;
+        const uint32_t last = room < kChunk ? (uint32_t)room : (uint32_t)kChunk;
+        const int32_t past32 = past < kChunk ? (int32_t)past : kChunk;
+        const TC *X = reinterpret_cast<const TC *>(a.x) + bb, *Y = reinterpret_cast<const TC *>(a.y) + bb;
+        const TV *V = reinterpret_cast<const TV *>(a.val) + (HAS_VAL ? bb : 0);
+        const uint8_t *C8 = reinterpret_cast<const uint8_t *>(a.cat.col) + (CK == CK_CODE8 ? bb : 0);
+        using VC = typename LoadVec<TC, kPer>::T;
+        using VV = typename LoadVec<TV, HAS_VAL ? kPer : 2>::T;
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            const uint32_t own = (uint32_t)(g * kPer * kScanThreads + kPer * tid);
+            const uint32_t off = own < last ? own : last;
+            shift[g] = past32 + (int32_t)(own - off);
+            const VC qx = __builtin_nontemporal_load(reinterpret_cast<const VC *>(X + off));
+            const VC qy = __builtin_nontemporal_load(reinterpret_cast<const VC *>(Y + off));
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) { x[g * kPer + i] = qx[i]; y[g * kPer + i] = qy[i]; }
+            if constexpr (HAS_VAL) {
+                const VV qv = __builtin_nontemporal_load(reinterpret_cast<const VV *>(V + off));
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) v[g * kPer + i] = qv[i];
             } else {
-                const int64_t rem = a.n - b;
-                lastq = rem >= kChunk ? (uint32_t)(kChunk / 4 - 1) : (uint32_t)(rem / 4 - 1);
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) v[g * kPer + i] = TV(0);
             }
-            const uint32_t q = (uint32_t)tid < lastq ? (uint32_t)tid : lastq;
-            const f32x4 X = stream_load(reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.x) + b) + q);
-            const f32x4 Y = stream_load(reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.y) + b) + q);
-            f32x4 V = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (HAS_VAL)
-                V = stream_load(reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.val) + b) + q);
-            uint32_t C4 = 0u;  // the four rows' one-byte codes (a 4-byte aligned column)
+            // (neighbouring waves' codes share cache lines: cached)
             if constexpr (CK == CK_CODE8)
-                C4 = reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(a.cat.col) + b)[q];
+                c8[g] = *reinterpret_cast<const typename LoadCodes<kPer>::T *>(C8 + off);
+            if constexpr (CK == CK_ANY) {
 #pragma unroll
-            for (int it = 0; it < kItems; ++it) {
-                x[it] = X[it];
-                y[it] = Y[it];
-                v[it] = HAS_VAL ? (TV)V[it] : TV(0);
-                c[it] = CK == CK_CODE8 ? (int64_t)((C4 >> (8 * it)) & 0xFFu) : 0;
+                for (int i = 0; i < kPer; ++i) c[g * kPer + i] = load_cat_raw(a.cat, bb + off + i);
             }
-            return;
-        }
-        // chunk base and last readable in-chunk row are uniform; each thread adds a
-        // 32-bit offset (scalar base + vector offset addressing)
-        int64_t b = ck * kChunk;
-        uint32_t lastj;
-        if (b >= a.n) {  // a prefetch past the end: re-read the last row
-            b = a.n > 0 ? a.n - 1 : 0;
-            lastj = 0;
-        } else {
-            const int64_t rem = a.n - b;
-            lastj = rem >= kChunk ? (uint32_t)(kChunk - 1) : (uint32_t)(rem - 1);
-        }
-        const TC *X = reinterpret_cast<const TC *>(a.x) + b;
-        const TC *Y = reinterpret_cast<const TC *>(a.y) + b;
-        const TV *V = reinterpret_cast<const TV *>(a.val) + (HAS_VAL ? b : 0);
-#pragma unroll
-        for (int it = 0; it < kItems; ++it) {
-            uint32_t j = (uint32_t)(it * kScanThreads + tid);
-            j = j < lastj ? j : lastj;
-            x[it] = stream_load(X + j);
-            y[it] = stream_load(Y + j);
-            if constexpr (HAS_VAL) v[it] = stream_load(V + j);
-            else v[it] = TV(0);
-            // (a byte column's 64-byte wave reads share cache lines between waves: cached)
-            if constexpr (CK == CK_BYTE || CK == CK_CODE8)
-                c[it] = reinterpret_cast<const uint8_t *>(a.cat.col)[b + j];
-            else if constexpr (CK == CK_ANY) c[it] = load_cat_raw(a.cat, b + j);
-            else c[it] = 0;
         }
     }
+    // whether row `it` is the thread's own, and its place in the chunk
+    __device__ __forceinline__ bool own(int it) const { return it % kPer >= shift[it / kPer]; }
+    __device__ __forceinline__ int32_t place(int it, int tid) const {
+        return it / kPer * kPer * kScanThreads + kPer * tid + it % kPer - shift[it / kPer];
+    }
+    __device__ __forceinline__ uint32_t code8(int it) const { return (c8[it / kPer] >> (8 * (it % kPer))) & 0xFFu; }
 };
+
+// Whether three sets of rows fit the registers of a scan: not the 64-bit category inputs
+// beside float64 coordinates and values (by(int32 codes, mean) over 20M rows, spread over
+// the canvas: 355 us a call with three sets, 307 with two).
+template <typename TC, typename TV, bool HAS_VAL, int CK>
+constexpr bool kDeepRows = !(CK == CK_ANY && sizeof(TC) == 8 && HAS_VAL && sizeof(TV) == 8);
+
+// A table of fewer than four rows as one of four, the rows after it without coordinates
+// (they are dropped): x, y, value and category columns at dst, 32 bytes apart.
+constexpr size_t kPadBytes = 128;
+__device__ __forceinline__ void pad_column(const void *src, uint8_t *dst, int n, int bytes, int tid,
+                                           bool nan) {
+    if (tid < 4 * bytes) {
+        const int r = tid / bytes;
+        dst[tid] = r < n && src ? reinterpret_cast<const uint8_t *>(src)[tid] : (nan ? 0xFF : 0);
+    }
+}
+__global__ void pad_rows_kernel(PointArgs a, uint8_t *dst, int cbytes, int vbytes, int catbytes) {
+    const int tid = threadIdx.x;
+    pad_column(a.x, dst, (int)a.n, cbytes, tid, true);
+    pad_column(a.y, dst + 32, (int)a.n, cbytes, tid, true);
+    pad_column(a.val, dst + 64, (int)a.n, vbytes, tid, true);
+    pad_column(a.cat.col, dst + 96, (int)a.n, catbytes, tid, false);
+}
+static int dtype_bytes(int32_t dt) {
+    switch (dt) {
+    case DSX_F64: case DSX_I64: return 8;
+    case DSX_I8: case DSX_U8: return 1;
+    case DSX_I16: return 2;
+    default: return 4;
+    }
+}
+// a's columns, or for fewer than four rows their padded copies in the workspace.
+static PointArgs pad_rows(const PointArgs &a, bool c64, int vbytes, uint8_t *ws, hipStream_t st) {
+    if (a.n >= 4) return a;
+    const int catbytes = a.cat.kind == DSX_CAT_NONE ? 1 : dtype_bytes(a.cat.dtype);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3(1), dim3(64), 0, st, a, ws, c64 ? 8 : 4, vbytes ? vbytes : 4,
+                       catbytes);
+    PointArgs p = a;
+    p.n = 4;
+    p.x = ws; p.y = ws + 32; p.val = ws + 64; p.cat.col = ws + 96;
+    return p;
+}
 
 // float64 to int32 by the hardware conversion (truncation; out-of-range values saturate,
 // NaN gives 0): defined for every input, so a row outside the view needs no select before
@@ -508,23 +549,50 @@ __device__ __forceinline__ uint32_t mul_add32(uint32_t a, uint32_t b, uint32_t c
     return m + c;
 }
 
-// Category of a scanned row from its loaded raw input; -1 when dropped.
-template <int CK>
-__device__ __forceinline__ int32_t scan_category(const Cat &c, int64_t raw) {
+// Category of a loaded row; -1 when dropped.
+template <int CK, typename R>
+__device__ __forceinline__ int32_t scan_category(const Cat &c, const R &rows, int it) {
     if constexpr (CK == CK_NONE) return 0;
     if constexpr (CK == CK_CODE8) {  // category_raw's codes branch, in 32 bits
-        int32_t k = c.dtype == DSX_I8 ? (int32_t)(int8_t)(uint8_t)raw : (int32_t)raw;
+        const uint32_t b8 = rows.code8(it);
+        int32_t k = c.dtype == DSX_I8 ? (int32_t)(int8_t)(uint8_t)b8 : (int32_t)b8;
         if (k < 0) k += c.ncat;
         return (uint32_t)k < (uint32_t)c.ncat ? k : -1;
     }
-    if constexpr (CK == CK_BYTE) raw = c.dtype == DSX_I8 ? (int64_t)(int8_t)(uint8_t)raw : raw;
-    return (int32_t)category_raw(c, raw);
+    return (int32_t)category_raw(c, rows.c[it]);
+}
+
+// Pixel of a loaded row, false when it is dropped.  LIN: locate_xy without branches, for a
+// view whose translation is exactly -xmin*sx, -ymin*sy (lin_view): an in-range row then
+// projects into [0, W] -- x >= xmin gives fl(x*sx) >= fl(xmin*sx) -- so the wraparound and
+// the lower bound never apply; a row out of range (NaN included) converts to anything
+// (cvt_sat_i32) and is dropped.
+template <bool LIN, typename R>
+__device__ __forceinline__ bool scan_pixel(const PointArgs &a, const R &rows, int it, int32_t &px,
+                                           int32_t &py) {
+    if constexpr (LIN) {
+        const double x = (double)rows.x[it], y = (double)rows.y[it];
+        const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
+        const int32_t xx = cvt_sat_i32(__dadd_rn(__dmul_rn(x, a.sx), a.tx));
+        const int32_t yy = cvt_sat_i32(__dadd_rn(__dmul_rn(y, a.sy), a.ty));
+        px = xx < a.W - 1 ? xx : a.W - 1;
+        py = yy < a.H - 1 ? yy : a.H - 1;
+        return rows.own(it) & inr;
+    } else {
+        px = py = 0;
+        return rows.own(it) && locate_xy(a, rows.x[it], rows.y[it], px, py);
+    }
+}
+
+static bool lin_view(const PointArgs &a) {
+    return !a.xlog && !a.ylog && a.sx > 0 && a.sy > 0 && a.tx == -(a.xmin * a.sx) &&
+           a.ty == -(a.ymin * a.sy);
 }
 
 // LIN: linear axes (no log10 call in the loop); WF: the window's plane set when known at
 // compile time (0: read from the layout).
 template <typename TC, typename TV, bool HAS_VAL, int KEYB, bool SQDEV, int CK, bool LIN = false,
-          uint32_t WF = 0, bool WIDE = false>
+          uint32_t WF = 0>
 __global__ __launch_bounds__(kScanThreads) void scan_kernel(PointArgs a, ScanArgs s) {
     if (tiles_run(s.window)) return;  // uniform: the tile strategy's scan runs instead
     extern __shared__ __align__(16) uint8_t smem[];
@@ -548,41 +616,21 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(PointArgs a, ScanArg
     // software pipeline, two chunks deep: while chunk ck is binned, the loads of chunks
     // ck + G and ck + 2G are in flight.  Three register sets rotate roles (binned / in
     // flight / being loaded), so no set is ever copied: a copy would wait for its loads.
-    using R = Rows<TC, TV, HAS_VAL, CK, WIDE>;
+    // (one chunk ahead where three sets spill registers: kDeepRows)
+    using R = Rows<TC, TV, HAS_VAL, CK>;
+    constexpr int kAhead = kDeepRows<TC, TV, HAS_VAL, CK> ? 2 : 1;
     R ra, rb, rc;
     ra.load(a, blockIdx.x, tid);
-    rb.load(a, (int64_t)blockIdx.x + gridDim.x, tid);
+    if constexpr (kAhead == 2) rb.load(a, (int64_t)blockIdx.x + gridDim.x, tid);
     int64_t ck = blockIdx.x;
     auto step = [&](R &cur, R &far) {
-        far.load(a, ck + 2 * (int64_t)gridDim.x, tid);
-        const int64_t rem64 = a.n - ck * kChunk;  // rows of this chunk, uniform
-        const uint32_t rem = rem64 >= kChunk ? (uint32_t)kChunk
-                                             : (rem64 > 0 ? (uint32_t)rem64 : 0u);
+        far.load(a, ck + kAhead * (int64_t)gridDim.x, tid);
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
-            // the row's place in the chunk (rows past rem are dropped)
-            const uint32_t j = WIDE ? (uint32_t)(4 * tid + it) : (uint32_t)(it * kScanThreads + tid);
-            int32_t px = 0, py = 0, pc = 0;
-            bool keep;
-            if constexpr (LIN) {
-                // locate_xy without branches, for a view whose translation is exactly
-                // -xmin*sx, -ymin*sy (checked on the host): an in-range row then projects
-                // into [0, W] -- x >= xmin gives fl(x*sx) >= fl(xmin*sx) -- so the
-                // wraparound and the lower bound never apply; a row out of range (NaN
-                // included) converts a harmless 0 and is dropped by `inr`
-                const double x = (double)cur.x[it], y = (double)cur.y[it];
-                const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
-                const double fx = inr ? __dadd_rn(__dmul_rn(x, a.sx), a.tx) : 0.0;
-                const double fy = inr ? __dadd_rn(__dmul_rn(y, a.sy), a.ty) : 0.0;
-                const int32_t xx = (int32_t)fx, yy = (int32_t)fy;
-                px = xx < a.W - 1 ? xx : a.W - 1;
-                py = yy < a.H - 1 ? yy : a.H - 1;
-                keep = (j < rem) & inr;
-            } else {
-                keep = j < rem && locate_xy<TC>(a, cur.x[it], cur.y[it], px, py);
-            }
+            int32_t px, py, pc = 0;
+            bool keep = scan_pixel<LIN>(a, cur, it, px, py);
             if constexpr (CK != CK_NONE) {
-                pc = scan_category<CK>(a.cat, cur.c[it]);
+                pc = scan_category<CK>(a.cat, cur, it);
                 keep = keep && pc >= 0;
             }
             const double v = HAS_VAL ? (double)cur.v[it] : 0.0;
@@ -645,11 +693,16 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(PointArgs a, ScanArg
     };
     // no exit between the three steps: a loop edge that skips steps makes the compiler's
     // wait counts assume fewer loads in flight, and it then drains the prefetch once per
-    // iteration.  Steps past the last chunk load the last row and keep nothing (rem = 0).
+    // iteration.  Steps past the last chunk load the last rows and keep nothing.
     while (ck < nchunks) {
-        step(ra, rc);
-        step(rb, ra);
-        step(rc, rb);
+        if constexpr (kAhead == 2) {
+            step(ra, rc);
+            step(rb, ra);
+            step(rc, rb);
+        } else {
+            step(ra, rb);
+            step(rb, ra);
+        }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if ((uint32_t)lane < staged) {  // the last partial line
@@ -1313,7 +1366,7 @@ constexpr int kBktOwn = 4;                      // buckets a thread owns (nb <= 
 static_assert(kBktOwn * kScanThreads >= kMaxTiles, "every bucket has an owner");
 constexpr int kBktSpare = 64;                   // spare bucket words (one per lane)
 
-template <typename TC, typename TV, bool HAS_VAL, int CK, bool LIN, bool WIDE = false>
+template <typename TC, typename TV, bool HAS_VAL, int CK, bool LIN>
 __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArgs s) {
     if (!tiles_run(s.rec)) return;  // uniform: the window strategy's scan runs instead
     constexpr int kSteps = (HAS_VAL || sizeof(TC) == 8) ? 1 : 3;  // chunks between checks
@@ -1509,14 +1562,14 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
         // check's barrier orders these writes before the next flush
     };
     const int64_t nchunks = (a.n + kChunk - 1) / kChunk;
-    using R = Rows<TC, TV, HAS_VAL, CK, WIDE>;
+    using R = Rows<TC, TV, HAS_VAL, CK>;
     // chunks loaded ahead: three where the checks come every three chunks (four register
     // sets: the loads in flight cover a flush), else two; the generic category column (a
     // 64-bit raw value a row) keeps two, as a fourth set would spill registers
-    constexpr int kAhead = (kSteps == 3 && CK != CK_ANY) ? 3 : 2;
+    constexpr int kAhead = !kDeepRows<TC, TV, HAS_VAL, CK> ? 1 : (kSteps == 3 && CK != CK_ANY) ? 3 : 2;
     R ra, rb, rc, rd;
     ra.load(a, blockIdx.x, tid);
-    rb.load(a, (int64_t)blockIdx.x + gridDim.x, tid);
+    if constexpr (kAhead >= 2) rb.load(a, (int64_t)blockIdx.x + gridDim.x, tid);
     if constexpr (kAhead == 3) rc.load(a, (int64_t)blockIdx.x + 2 * (int64_t)gridDim.x, tid);
     int64_t ck = blockIdx.x;
     uint32_t fk = 0;  // this check's flag: ctrl[2 + fk]
@@ -1524,9 +1577,6 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
     // pb: the first of this chunk's kItems entries of pend (a constant at every call)
     auto step = [&](R &cur, R &far, const int pb) {
         far.load(a, ck + kAhead * (int64_t)gridDim.x, tid);
-        const int64_t rem64 = a.n - ck * kChunk;
-        const uint32_t rem = rem64 >= kChunk ? (uint32_t)kChunk
-                                             : (rem64 > 0 ? (uint32_t)rem64 : 0u);
         // three passes over the chunk's rows, so that the LDS round trips of all its rows
         // are in flight together: bin every row (a dropped row takes its lane's spare
         // bucket, whose slots are never stored), take every slot, then store
@@ -1534,28 +1584,15 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
         uint16_t oo[kItems];
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
-            const uint32_t j = WIDE ? (uint32_t)(4 * tid + it) : (uint32_t)(it * kScanThreads + tid);
-            int32_t px = 0, py = 0, pc = 0;
-            bool keep;
-            if constexpr (LIN) {  // as in scan_kernel, without its selects (cvt_sat_i32)
-                const double x = (double)cur.x[it], y = (double)cur.y[it];
-                const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
-                const double fx = __dadd_rn(__dmul_rn(x, a.sx), a.tx);
-                const double fy = __dadd_rn(__dmul_rn(y, a.sy), a.ty);
-                const int32_t xx = cvt_sat_i32(fx), yy = cvt_sat_i32(fy);
-                px = xx < a.W - 1 ? xx : a.W - 1;
-                py = yy < a.H - 1 ? yy : a.H - 1;
-                keep = (j < rem) & inr;
-            } else {
-                keep = j < rem && locate_xy<TC>(a, cur.x[it], cur.y[it], px, py);
-            }
+            int32_t px, py, pc = 0;
+            bool keep = scan_pixel<LIN>(a, cur, it, px, py);
             if constexpr (CK == CK_CODE8) {
-                const uint32_t b8 = (uint32_t)cur.c[it];
+                const uint32_t b8 = cur.code8(it);
                 const uint32_t k = b8 - (b8 >= c8_at ? c8_sub : 0u);
                 keep = keep & (k < (uint32_t)ncat);
                 pc = (int32_t)k;
             } else if constexpr (CK != CK_NONE) {
-                pc = scan_category<CK>(a.cat, cur.c[it]);
+                pc = scan_category<CK>(a.cat, cur, it);
                 keep = keep && pc >= 0;
             }
             // cells < 2^32 (checked on the host), so 32-bit arithmetic is exact; py, W ncat,
@@ -1602,6 +1639,12 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
             step(rd, rc, 0); step(ra, rd, kItems); step(rb, ra, 2 * kItems); check();
             step(rc, rb, 0); step(rd, rc, kItems); step(ra, rd, 2 * kItems); check();
             step(rb, ra, 0); step(rc, rb, kItems); step(rd, rc, 2 * kItems); check();
+        }
+    } else if constexpr (kAhead == 1) {
+        static_assert(kSteps == 1, "a check after every chunk");
+        while (ck < nchunks) {
+            step(ra, rb, 0); check();
+            step(rb, ra, 0); check();
         }
     } else {
         while (ck < nchunks) {  // three steps per trip, as in scan_kernel
@@ -1828,7 +1871,7 @@ struct Plan {
     size_t scan_lds, tile_lds;
     uint32_t o_thist, o_stage_cell, o_stage_val;  // scan LDS offsets
     // workspace offsets
-    size_t o_window, o_hist_sel, o_count, o_partials, o_spill_cell, o_spill_val, o_hist,
+    size_t o_window, o_pad, o_hist_sel, o_count, o_partials, o_spill_cell, o_spill_val, o_hist,
         o_totals, o_tile_start, o_sorted_cell, o_sorted_val, o_part_start, o_part_len, o_part_tile,
         o_scratch, total;
     int32_t max_parts;   // upper bound of the tile parts (grid of the tile kernel)
@@ -1981,6 +2024,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     const int64_t n = d->n < 1 ? 1 : d->n;
     size_t o = 0;
     P.o_window = o; o = align_up(o + 4 * kRecWords, 256);
+    P.o_pad = o; o = align_up(o + kPadBytes, 256);
     P.o_hist_sel = o; o = align_up(o + 4 * (size_t)kSelBins, 256);
     P.o_count = o; o = align_up(o + 4 * (size_t)P.scan_groups * kWaves, 256);  // sub-segment lengths
     P.o_hist = o; o = align_up(o + 4 * (size_t)P.scan_groups * P.ntiles, 256);
@@ -2069,25 +2113,16 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     sa.o_stage_val = P.o_stage_val;
     sa.spill_nan = (P.flags & PL_NAN) ? 1u : 0u;
     sa.mean = mean;
-    // the scan reads row 0 of each column even for an empty input (and drops it): give
-    // an empty input a readable dummy row in the workspace
-    PointArgs sa_a = a;
-    if (a.n == 0) {
-        sa_a.x = sa_a.y = sa_a.val = hist_sel;
-        sa_a.cat.col = hist_sel;
-    }
+    const PointArgs sa_a = pad_rows(a, sizeof(TC) == 8, HAS_VAL ? (int)sizeof(TV) : 0, ws + P.o_pad, st);
+    const int ck = cat_kind(a.cat);
+    const bool lin = lin_view(a);
     auto scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_ANY>;
-    if (a.cat.kind == DSX_CAT_NONE) scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE>;
-    else if ((a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8) && a.cat.kind == DSX_CAT_CODES)
-        scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_CODE8>;
-    else if (a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8)
-        scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_BYTE>;
+    if (ck == CK_NONE) scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE>;
+    else if (ck == CK_CODE8) scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_CODE8>;
     // the common plane sets over linear axes, without categorizer: compile-time planes
     // (the linear fast path also needs the reference's own translation, t = -start * s,
     // under which in-range rows cannot project below pixel 0)
-    const bool origin = a.sx > 0 && a.sy > 0 && a.tx == -(a.xmin * a.sx) &&
-                        a.ty == -(a.ymin * a.sy);
-    if (a.cat.kind == DSX_CAT_NONE && !a.xlog && !a.ylog && origin) {
+    if (ck == CK_NONE && lin) {
         const uint32_t wf = P.wl.flags;
         if constexpr (!HAS_VAL) {
             if (wf == PL_CNT) scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNT>;
@@ -2100,22 +2135,6 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
                 scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNTV | PL_SUM>;
             else if (wf == PL_CNT)
                 scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNT>;
-        }
-        // float32 columns, 16-byte aligned, whole groups of four rows: the wide loads
-        const bool wide = sizeof(TC) == 4 && (!HAS_VAL || sizeof(TV) == 4) && d->n >= 4 &&
-                          d->n % 4 == 0 && ((uintptr_t)a.x % 16) == 0 && ((uintptr_t)a.y % 16) == 0 &&
-                          (!HAS_VAL || ((uintptr_t)a.val % 16) == 0);
-        if constexpr (sizeof(TC) == 4 && (!HAS_VAL || sizeof(TV) == 4)) {
-            if (wide) {
-                if constexpr (!HAS_VAL) {
-                    if (wf == PL_CNT) scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNT, true>;
-                } else if constexpr (!SQDEV) {
-                    if (wf == (PL_CNT | PL_SUM))
-                        scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNT | PL_SUM, true>;
-                    else if (wf == (PL_CNTV | PL_SUM))
-                        scan = scan_kernel<TC, TV, HAS_VAL, KEYB, SQDEV, CK_NONE, true, PL_CNTV | PL_SUM, true>;
-                }
-            }
         }
     }
     hipError_t e;
@@ -2152,28 +2171,13 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
         ba.o_ctrl = P.bo_ctrl;
         ba.loc_cap = P.bo_cnt / 4u;  // values and offsets come first, from byte 0
         ba.batch = P.batch;
-        const bool lin = !a.xlog && !a.ylog && origin;
         auto bscan = bscan_kernel<TC, TV, HAS_VAL, CK_ANY, false>;
-        if (a.cat.kind == DSX_CAT_NONE)
+        if (ck == CK_NONE)
             bscan = lin ? bscan_kernel<TC, TV, HAS_VAL, CK_NONE, true>
                         : bscan_kernel<TC, TV, HAS_VAL, CK_NONE, false>;
-        else if ((a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8) && a.cat.kind == DSX_CAT_CODES)
+        else if (ck == CK_CODE8)
             bscan = lin ? bscan_kernel<TC, TV, HAS_VAL, CK_CODE8, true>
                         : bscan_kernel<TC, TV, HAS_VAL, CK_CODE8, false>;
-        // float32 columns without values, 16-byte aligned (the code column 4-byte aligned),
-        // whole groups of four rows: the wide loads
-        if constexpr (sizeof(TC) == 4 && !HAS_VAL) {
-            const bool codes = (a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8) &&
-                               a.cat.kind == DSX_CAT_CODES;
-            const bool wide = lin && d->n >= 4 && d->n % 4 == 0 && ((uintptr_t)a.x % 16) == 0 &&
-                              ((uintptr_t)a.y % 16) == 0 &&
-                              (a.cat.kind == DSX_CAT_NONE || (codes && ((uintptr_t)a.cat.col % 4) == 0));
-            if (wide)
-                bscan = a.cat.kind == DSX_CAT_NONE ? bscan_kernel<TC, TV, HAS_VAL, CK_NONE, true, true>
-                                                   : bscan_kernel<TC, TV, HAS_VAL, CK_CODE8, true, true>;
-        }
-        else if (a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8)
-            bscan = bscan_kernel<TC, TV, HAS_VAL, CK_BYTE, false>;
         e = hipFuncSetAttribute((const void *)bscan, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)P.bscan_lds);
         if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
@@ -2809,31 +2813,15 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
     const int64_t nchunks = (a.n + kChunk - 1) / kChunk;
     using R = Rows<TC, TV, true, CK>;
     auto step = [&](int64_t ck, const R &S, R &far) {
-        const int64_t b = ck * kChunk;
-        const int64_t rem64 = a.n - b;
-        const uint32_t rem = rem64 >= kChunk ? (uint32_t)kChunk : (rem64 > 0 ? (uint32_t)rem64 : 0u);
         int64_t cell[kItems];
         bool keep[kItems];
         typename K::T kv[kItems];
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
-            const uint32_t j = (uint32_t)(it * kScanThreads + tid);
-            int32_t px = 0, py = 0, pc = 0;
-            bool k_;
-            if constexpr (LIN) {  // as in scan_kernel
-                const double x = (double)S.x[it], y = (double)S.y[it];
-                const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
-                const double fx = inr ? __dadd_rn(__dmul_rn(x, a.sx), a.tx) : 0.0;
-                const double fy = inr ? __dadd_rn(__dmul_rn(y, a.sy), a.ty) : 0.0;
-                const int32_t xx = (int32_t)fx, yy = (int32_t)fy;
-                px = xx < a.W - 1 ? xx : a.W - 1;
-                py = yy < a.H - 1 ? yy : a.H - 1;
-                k_ = (j < rem) & inr;
-            } else {
-                k_ = j < rem && locate_xy<TC>(a, S.x[it], S.y[it], px, py);
-            }
+            int32_t px, py, pc = 0;
+            bool k_ = scan_pixel<LIN>(a, S, it, px, py);
             if constexpr (CK != CK_NONE) {
-                pc = scan_category<CK>(a.cat, S.c[it]);
+                pc = scan_category<CK>(a.cat, S, it);
                 k_ = k_ && pc >= 0;
             }
             k_ = k_ && !(S.v[it] != S.v[it]);
@@ -2846,7 +2834,7 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             if (!keep[it] || K::key((double)S.v[it]) != kv[it]) continue;
-            const unsigned long long row = (unsigned long long)(b + it * kScanThreads + tid);
+            const unsigned long long row = (unsigned long long)(ck * kChunk + S.place(it, tid));
             __hip_atomic_fetch_min(index + cell[it], row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
@@ -2864,12 +2852,9 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
 template <typename TC>
 static int rowindex_launch(const RiArgs &r, int val_dtype, hipStream_t st) {
     const bool arg = r.mode == DSX_RI_ARGMAX || r.mode == DSX_RI_ARGMIN;
-    if (arg) {  // the streaming form
+    if (arg && r.a.n >= 4) {  // the streaming form
         const PointArgs &a = r.a;
-        const bool lin = !a.xlog && !a.ylog && a.sx > 0 && a.sy > 0 &&
-                         a.tx == -(a.xmin * a.sx) && a.ty == -(a.ymin * a.sy);
-        const bool byte = (a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8) &&
-                          a.cat.kind == DSX_CAT_CODES;
+        const bool lin = lin_view(a), byte = cat_kind(a.cat) == CK_CODE8;
         const int64_t chunks = (a.n + kChunk - 1) / kChunk;
         const int groups = grid_for(chunks < 1 ? 1 : chunks, 1, 1);  // one per CU at most
         auto kern = rowindex_arg_kernel<TC, double, CK_ANY, false>;
@@ -2933,7 +2918,7 @@ struct RiwArgs {
 struct RiwPlan {
     uint32_t cap;
     int groups, bshift, cw, ch;
-    size_t lds, o_window, o_hist, o_partials, total;
+    size_t lds, o_window, o_pad, o_hist, o_partials, total;
 };
 
 static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, bool packed = false,
@@ -2960,6 +2945,7 @@ static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, boo
     P.ch = (v->height + (1 << P.bshift) - 1) >> P.bshift;
     size_t o = 0;
     P.o_window = o; o = align_up(o + 4 * kRecWords, 256);
+    P.o_pad = o; o = align_up(o + kPadBytes, 256);
     P.o_hist = o; o = align_up(o + 4 * (size_t)kSelBins, 256);
     P.o_partials = o; o = align_up(o + cb * (size_t)P.cap * (size_t)P.groups, 256);
     P.total = o;
@@ -2969,7 +2955,7 @@ static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, boo
 // NANCHK: rows whose value is NaN are skipped (the value column is read); CK, LIN: as
 // in scan_kernel (the category read with the row's other columns, the branch-free linear
 // projection); PK: the packed ARGMAX / ARGMIN form (float32 values).
-template <typename TC, typename TV, bool NANCHK, int CK, bool LIN, bool PK = false, bool WIDE = false>
+template <typename TC, typename TV, bool NANCHK, int CK, bool LIN, bool PK = false>
 __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r) {
     static_assert(kRiwThreads == kScanThreads && kRiwItems == kItems, "chunks as the scan's");
     static_assert(!PK || sizeof(TV) == 4, "packed: float32 values");
@@ -3005,7 +2991,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     // that after the first sweep most rows fail the global skip test; a step past the
     // last chunk reads chunk nchunks (rows past the end: re-reads the last row, dropped)
     auto chunk_of = [&](int64_t k) { return k >= nchunks ? nchunks : (r.last ? nchunks - 1 - k : k); };
-    using R = Rows<TC, TV, NANCHK, CK, WIDE>;
+    using R = Rows<TC, TV, NANCHK, CK>;
     auto *const index = global_ptr(r.index);
     auto *const sindex = global_ptr(reinterpret_cast<long long *>(r.index));
     // Three register sets rotate roles (binned / in flight / being loaded), as in the
@@ -3016,9 +3002,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     // for those loads.
     auto step = [&](int64_t k, const R &S, R &far) {
         const int64_t ck = chunk_of(k);
-        const int64_t b = ck * kChunk;
-        const int64_t rem64 = a.n - b;
-        const uint32_t rem = rem64 >= kChunk ? (uint32_t)kChunk : (rem64 > 0 ? (uint32_t)rem64 : 0u);
+        const int64_t row0 = ck * kChunk;
         int64_t cell[kRiwItems];
         long long cur[kRiwItems];
         unsigned long long pkv[kRiwItems];  // PK: the row's packed value
@@ -3026,31 +3010,17 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
         bool out[kRiwItems];
 #pragma unroll
         for (int it = 0; it < kRiwItems; ++it) {
-            // the row's place in the chunk: as the loader placed it
-            const uint32_t j = WIDE ? (uint32_t)(4 * tid + it) : (uint32_t)(it * kRiwThreads + tid);
-            int32_t px = 0, py = 0, pc = 0;
-            bool keep;
-            if constexpr (LIN) {  // as in scan_kernel
-                const double x = (double)S.x[it], y = (double)S.y[it];
-                const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
-                const double fx = inr ? __dadd_rn(__dmul_rn(x, a.sx), a.tx) : 0.0;
-                const double fy = inr ? __dadd_rn(__dmul_rn(y, a.sy), a.ty) : 0.0;
-                const int32_t xx = (int32_t)fx, yy = (int32_t)fy;
-                px = xx < a.W - 1 ? xx : a.W - 1;
-                py = yy < a.H - 1 ? yy : a.H - 1;
-                keep = (j < rem) & inr;
-            } else {
-                keep = j < rem && locate_xy<TC>(a, S.x[it], S.y[it], px, py);
-            }
+            int32_t px, py, pc = 0;
+            bool keep = scan_pixel<LIN>(a, S, it, px, py);
             if constexpr (CK != CK_NONE) {
-                pc = scan_category<CK>(a.cat, S.c[it]);
+                pc = scan_category<CK>(a.cat, S, it);
                 keep = keep && pc >= 0;
             }
             if constexpr (NANCHK) keep = keep && !(S.v[it] != S.v[it]);
             out[it] = false;
             cell[it] = 0;
             cur[it] = 0;
-            const uint32_t row = (uint32_t)(b + j);  // rows < 2^32 (checked on the host)
+            const uint32_t row = (uint32_t)(row0 + S.place(it, tid));  // rows < 2^32 (checked on the host)
             pkv[it] = 0ull;
             pth[it] = 0ull;
             if constexpr (PK)
@@ -3098,8 +3068,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
                 }
                 continue;
             }
-            const long long row =
-                (long long)(b + (WIDE ? 4 * tid + it : it * kRiwThreads + tid));
+            const long long row = (long long)(row0 + S.place(it, tid));
             if (r.last) {
                 if (row > cur[it])
                     __hip_atomic_fetch_max(sindex + cell[it], row, __ATOMIC_RELAXED,
@@ -3220,11 +3189,10 @@ static int riw_launch(const dsx_points_desc *d, const RiwArgs &r, const RiwPlan 
     if ((s = launch_status())) return s;
     // (the linear fast path needs the reference's own translation, as in the points scan)
     const PointArgs &a = r.a;
-    const bool lin = !a.xlog && !a.ylog && a.sx > 0 && a.sy > 0 && a.tx == -(a.xmin * a.sx) &&
-                     a.ty == -(a.ymin * a.sy);
+    const bool lin = lin_view(a);
     const bool f32v = d->val_dtype == DSX_F32;
     const bool nan = r.nan_check != 0;
-    const bool byte = (a.cat.dtype == DSX_I8 || a.cat.dtype == DSX_U8) && a.cat.kind == DSX_CAT_CODES;
+    const bool byte = cat_kind(a.cat) == CK_CODE8;
     auto kern = rowindex_window_kernel<TC, double, false, CK_ANY, false>;
     if (a.cat.kind == DSX_CAT_NONE) {
         if (lin) kern = nan ? (f32v ? rowindex_window_kernel<TC, float, true, CK_NONE, true>
@@ -3255,25 +3223,12 @@ static int riw_launch(const dsx_points_desc *d, const RiwArgs &r, const RiwPlan 
         else if (byte) kern = rowindex_window_kernel<TC, float, false, CK_CODE8, false, true>;
         else kern = rowindex_window_kernel<TC, float, false, CK_ANY, false, true>;
     }
-    // float32 columns, 16-byte aligned, whole groups of four rows, linear axes, no
-    // categorizer: the wide row loads
-    if constexpr (sizeof(TC) == 4) {
-        const bool wide = lin && a.cat.kind == DSX_CAT_NONE && d->n >= 4 && d->n % 4 == 0 &&
-                          ((uintptr_t)a.x % 16) == 0 && ((uintptr_t)a.y % 16) == 0 &&
-                          (!nan || (f32v && ((uintptr_t)a.val % 16) == 0));
-        if (wide) {
-            if (r.packed)
-                kern = nan ? rowindex_window_kernel<TC, float, true, CK_NONE, true, true, true>
-                           : rowindex_window_kernel<TC, float, false, CK_NONE, true, true, true>;
-            else
-                kern = nan ? rowindex_window_kernel<TC, float, true, CK_NONE, true, false, true>
-                           : rowindex_window_kernel<TC, double, false, CK_NONE, true, false, true>;
-        }
-    }
     const hipError_t e = hipFuncSetAttribute((const void *)kern,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
     if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-    hipLaunchKernelGGL(kern, dim3(P.groups), dim3(kRiwThreads), P.lds, st, r);
+    RiwArgs rk = r;
+    rk.a = pad_rows(r.a, sizeof(TC) == 8, nan ? (f32v ? 4 : 8) : 0, ws + P.o_pad, st);
+    hipLaunchKernelGGL(kern, dim3(P.groups), dim3(kRiwThreads), P.lds, st, rk);
     if ((s = launch_status())) return s;
     hipLaunchKernelGGL(rowindex_window_merge, dim3(grid_for(P.cap, 256, 4)), dim3(256), 0, st, r,
                        P.groups);
