@@ -30,7 +30,8 @@ FILL_ZERO32, FILL_ONES32, FILL_ZERO64, FILL_ONES64 = 1, 2, 3, 4
 # finalize modes
 FIN_ANY, FIN_SUM, FIN_MEAN, FIN_VAR, FIN_STD, FIN_MIN, FIN_MAX, FIN_SUMZERO = range(1, 9)
 
-EXPORTS = ("dsx_points_workspace_size", "dsx_points_agg", "dsx_lines_agg",
+EXPORTS = ("dsx_points_workspace_size", "dsx_points_agg", "dsx_points_m2_workspace_size",
+           "dsx_points_agg_m2", "dsx_lines_agg",
            "dsx_bounds_workspace_size", "dsx_bounds", "dsx_bounds_noalloc", "dsx_fill", "dsx_finalize",
            "dsx_grid_index_workspace_size", "dsx_grid_index_build", "dsx_gather_rows",
            "dsx_points_indexed_workspace_size", "dsx_points_agg_indexed",
@@ -195,6 +196,9 @@ def load():
         lib.dsx_points_workspace_size.argtypes = [P(PointsDesc), P(View), P(Planes)]
         lib.dsx_points_workspace_size.restype = sz
         lib.dsx_points_agg.argtypes = [P(PointsDesc), P(View), P(Planes), vp, vp, sz, vp]
+        lib.dsx_points_m2_workspace_size.argtypes = [P(PointsDesc), P(View), P(Planes)]
+        lib.dsx_points_m2_workspace_size.restype = sz
+        lib.dsx_points_agg_m2.argtypes = [P(PointsDesc), P(View), P(Planes), vp, vp, sz, vp]
         lib.dsx_lines_agg.argtypes = [P(LinesDesc), P(View), P(Planes), vp]
         lib.dsx_bounds_workspace_size.argtypes = [i64]
         lib.dsx_bounds_workspace_size.restype = sz
@@ -238,7 +242,7 @@ def load():
         lib.dsx_strerror.restype = ctypes.c_char_p
         lib.dsx_last_hip_error.argtypes = []
         lib.dsx_last_hip_error.restype = ctypes.c_char_p
-        for f in ("dsx_points_agg", "dsx_lines_agg", "dsx_bounds", "dsx_bounds_noalloc", "dsx_fill", "dsx_finalize",
+        for f in ("dsx_points_agg", "dsx_points_agg_m2", "dsx_lines_agg", "dsx_bounds", "dsx_bounds_noalloc", "dsx_fill", "dsx_finalize",
                   "dsx_grid_index_build", "dsx_gather_rows", "dsx_points_agg_indexed",
                   "dsx_shade", "dsx_combine", "dsx_points_rowindex", "dsx_take",
                   "dsx_points_nselect", "dsx_batch_create", "dsx_batch_submit",

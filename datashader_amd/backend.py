@@ -229,10 +229,20 @@ def _grid_ref(frame, glyph, p, view):
     return r
 
 
-def _points_call(lib, d, vw, planes_struct, mean, device, stream, grid=None):
-    """dsx_points_agg (or, over an indexed frame, dsx_points_agg_indexed) with a
-    workspace from torch's caching allocator."""
+def _points_call(lib, d, vw, planes_struct, mean, device, stream, grid=None, m2=None):
+    """dsx_points_agg (or, over an indexed frame, dsx_points_agg_indexed; with an m2 plane,
+    dsx_points_agg_m2) with a workspace from torch's caching allocator."""
     t = dev.torch()
+    if m2 is not None:
+        ws = int(lib.dsx_points_m2_workspace_size(d, vw, planes_struct))
+        if ws == 0:
+            raise _abi.DsxError("dsx_points_m2_workspace_size rejected the call (invalid "
+                                "descriptor or shape)")
+        work = t.empty(ws, dtype=t.uint8, device=device)
+        _abi.check(_timed(lambda: lib.dsx_points_agg_m2(d, vw, planes_struct, dev.ptr(m2),
+                                                        dev.ptr(work), ws, stream)),
+                   "dsx_points_agg_m2")
+        return
     ws = int(lib.dsx_points_indexed_workspace_size(d, vw, planes_struct, grid)) if grid else 0
     if grid is not None and ws > 0:  # a view the lattice tiles cannot take: plain call
         work = t.empty(ws, dtype=t.uint8, device=device)
@@ -358,6 +368,9 @@ def run_pass(lib, frame, schema, glyph, view, p, H, W, with_m2=True, fuse_mean=T
     grid = None
     if points:
         grid = _grid_ref(frame, glyph, p, view)
+        m2 = None
+        if p.m2 and with_m2 and "mean" in planes and grid is None:  # both passes in one call
+            m2 = planes["m2"] = _alloc(ncells, "f64", device)
         if grid is None and getattr(frame, "persistent", False):
             key = (glyph.x, glyph.y, p.val, None if p.cat is None else p.cat._key(),
                    tuple(sorted(p.planes)),
@@ -366,13 +379,13 @@ def run_pass(lib, frame, schema, glyph, view, p, H, W, with_m2=True, fuse_mean=T
             d.window, d.reuse_window = dev.ptr(slot.rec), reuse
             if FORCE_STRATEGY is None:
                 d.strategy = strategy
-            _points_call(lib, d, vw, ps, None, device, stream, grid)
+            _points_call(lib, d, vw, ps, None, device, stream, grid, m2)
             _window_readback(slot)
         else:
-            _points_call(lib, d, vw, ps, None, device, stream, grid)
+            _points_call(lib, d, vw, ps, None, device, stream, grid, m2)
     else:
         _abi.check(_timed(lambda: lib.dsx_lines_agg(d, vw, ps, stream)), "dsx_lines_agg")
-    if p.m2 and with_m2:
+    if p.m2 and with_m2 and "m2" not in planes:
         if "mean" in planes:
             mean = planes["mean"]
         else:

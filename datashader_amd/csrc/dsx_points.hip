@@ -226,11 +226,14 @@ __device__ __forceinline__ bool in_window(const Window &w, int32_t px, int32_t p
 // A call's window record: {x0, y0, w, h, strategy, 0, 0, 0} (kRecWords int32 words).
 constexpr int kRecWords = 8;
 
+// (skip: as for select_pick_kernel)
 __global__ void set_window_kernel(int32_t *w, int32_t x0, int32_t y0, int32_t ww, int32_t wh,
-                                  int32_t strategy) {
+                                  int32_t strategy, const int32_t *skip) {
     if (threadIdx.x < kRecWords) {
+        const bool none = skip && skip[4] == DSX_STRATEGY_TILES;
         const int32_t r[4] = {x0, y0, ww, wh};
-        w[threadIdx.x] = threadIdx.x < 4 ? r[threadIdx.x] : (threadIdx.x == 4 ? strategy : 0);
+        w[threadIdx.x] = threadIdx.x == 4 ? (none ? DSX_STRATEGY_TILES : strategy)
+                                          : (threadIdx.x < 4 && !none ? r[threadIdx.x] : 0);
     }
 }
 
@@ -252,7 +255,8 @@ __device__ __forceinline__ bool tiles_run(const int32_t *rec) {
 template <typename TC>
 __global__ __launch_bounds__(1024) void select_hist_kernel(PointArgs a, int32_t bshift,
                                                            int32_t cw, int32_t ch,
-                                                           uint32_t *hist) {
+                                                           uint32_t *hist, const int32_t *skip) {
+    if (skip && tiles_run(skip)) return;  // uniform: no window is wanted
     __shared__ uint32_t h[kSelBins];
     for (int b = threadIdx.x; b < kSelBins; b += blockDim.x) h[b] = 0u;
     __syncthreads();
@@ -281,7 +285,12 @@ __global__ __launch_bounds__(1024) void select_hist_kernel(PointArgs a, int32_t 
 __global__ __launch_bounds__(1024) void select_pick_kernel(const uint32_t *hist, int32_t bshift,
                                                            int32_t cw, int32_t ch, int32_t W,
                                                            int32_t H, int64_t cap_px,
-                                                           int32_t tiles_ok, int32_t *win) {
+                                                           int32_t tiles_ok, int32_t *win,
+                                                           const int32_t *skip) {
+    if (skip && tiles_run(skip)) {  // uniform: the tile strategy, as the record `skip` has it
+        if (threadIdx.x < kRecWords) win[threadIdx.x] = threadIdx.x == 4 ? DSX_STRATEGY_TILES : 0;
+        return;
+    }
     // (cw+1) x (ch+1) inclusive prefix sums; cw*ch <= kSelBins, so cw + ch <= kSelBins + 1
     __shared__ uint32_t ps[2 * kSelBins + 2];
     __shared__ unsigned long long best[1024 / 64];
@@ -834,6 +843,7 @@ struct PartArgs {
     uint32_t *part_len;               // [1]
     uint8_t *scratch;                 // one tile-layout region per part of a split tile
     const int32_t *rec;               // the call's window record (its strategy)
+    int32_t window_only;              // no tables under the tile strategy (a skipped call)
     uint32_t min_part_tiles;          // fewest blocks a tile part is given (tile strategy)
 };
 
@@ -900,6 +910,7 @@ __device__ __forceinline__ uint32_t block_exscan32(uint32_t v, uint32_t *sh, uin
 // place, and the tile total.
 __global__ __launch_bounds__(kPartThreads) void spill_colscan_kernel(PartArgs p,
                                                                     unsigned long long *totals) {
+    if (p.window_only && tiles_run(p.rec)) return;  // uniform
     __shared__ unsigned long long sh[kPartThreads / 64 + 1];
     const int t = blockIdx.x;
     const int g = threadIdx.x;  // ngroups <= kPartThreads
@@ -912,6 +923,7 @@ __global__ __launch_bounds__(kPartThreads) void spill_colscan_kernel(PartArgs p,
 
 __global__ __launch_bounds__(kPartThreads) void spill_tilescan_kernel(PartArgs p,
                                                                      const unsigned long long *totals) {
+    if (p.window_only && tiles_run(p.rec)) return;  // uniform
     __shared__ unsigned long long sh[kPartThreads / 64 + 1];
     unsigned long long carry = 0;
     for (int t0 = 0; t0 < p.ntiles; t0 += blockDim.x) {
@@ -1297,10 +1309,13 @@ __global__ __launch_bounds__(kTileThreads) void tile_merge_kernel(PartArgs p, La
                                                                  const int32_t *window, int32_t W,
                                                                  int32_t H, int64_t wcap_px,
                                                                  int32_t ncat, int64_t ncells,
-                                                                 Planes out) {
+                                                                 Planes out, int32_t only) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int t = blockIdx.x;
-    if (t >= p.ntiles) return;
+    // only: the strategy whose tiles these are (0: the one that ran)
+    if (t >= p.ntiles || (only == DSX_STRATEGY_TILES && !tiles_run(window)) ||
+        (only == DSX_STRATEGY_WINDOW && tiles_run(window)))
+        return;
     const uint32_t first = p.part_start[t], nparts = p.part_start[t + 1] - first;
     if (nparts <= 1) return;  // uniform
     fold_parts<kTileThreads, KEYB>(smem, L, p.scratch + (size_t)first * L.bytes, nparts);
@@ -1891,6 +1906,24 @@ struct Plan {
 
 static size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// LDS of the tile strategy's scan: nb buckets of C entries, values of vb bytes.
+static size_t bkt_layout(size_t vb, size_t nb, size_t C, Plan &P) {
+    size_t q = 0;
+    P.bo_val = (uint32_t)q; q = align_up(q + vb * C * nb, 16);   // values first (8-aligned)
+    P.bo_off = (uint32_t)q; q = align_up(q + 2 * C * nb, 16);
+    P.bo_cnt = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
+    P.bo_lo = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
+    P.bo_tblk = (uint32_t)q; q = align_up(q + 4 * nb, 16);
+    P.bo_base = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
+    // (the end's scan scratch, >= 17 words; during the scan, a spare offset and value
+    // position for each lane of a wave)
+    P.bo_bk = (uint32_t)q; q = align_up(q + 8 * 64, 16);
+    // (the end-of-scan list; during the scan, the flushes' per-wave lists)
+    P.bo_fl = (uint32_t)q; q = align_up(q + 8 * (nb > (size_t)kScanThreads ? nb : (size_t)kScanThreads), 16);
+    P.bo_ctrl = (uint32_t)q; q += 32;
+    return q;
+}
+
 static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *pl, Plan &P) {
     if (plane_flags(pl) == 0) return DSX_ERR_ACCUM;
     P.flags = internal_flags(plane_flags(pl));
@@ -1977,19 +2010,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
         for (int cs = 8; (1 << cs) >= kBktMinC && !P.tiles_ok; --cs) {
             if ((1 << cs) > kBktMaxC) continue;
             const size_t C = (size_t)1 << cs;
-            size_t q = 0;
-            P.bo_val = (uint32_t)q; q = align_up(q + vb * C * nb, 16);   // values first (8-aligned)
-            P.bo_off = (uint32_t)q; q = align_up(q + 2 * C * nb, 16);
-            P.bo_cnt = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
-            P.bo_lo = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
-            P.bo_tblk = (uint32_t)q; q = align_up(q + 4 * nb, 16);
-            P.bo_base = (uint32_t)q; q = align_up(q + 4 * (nb + kBktSpare), 16);
-            // (the end's scan scratch, >= 17 words; during the scan, a spare offset and
-            // value position for each lane of a wave)
-            P.bo_bk = (uint32_t)q; q = align_up(q + 8 * 64, 16);
-            // (the end-of-scan list; during the scan, the flushes' per-wave lists)
-            P.bo_fl = (uint32_t)q; q = align_up(q + 8 * (nb > (size_t)kScanThreads ? nb : (size_t)kScanThreads), 16);
-            P.bo_ctrl = (uint32_t)q; q += 32;
+            const size_t q = bkt_layout(vb, nb, C, P);
             const int64_t bcap = (group_rows + (int64_t)C - 1) / (int64_t)C + (int64_t)nb;
             // (512 bytes left for the kernel's static LDS words)
             if (q <= (size_t)kLdsBytes - 512 && (int64_t)P.scan_groups * bcap < (1ll << 32)) {
@@ -2060,9 +2081,21 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     return DSX_OK;
 }
 
+template <typename TC, typename TV, int KEYB>
+static int run_window_m2(const dsx_points_desc *d, const PointArgs &a, const Plan &P1, const double *mean,
+                         double *m2, uint8_t *ws, hipStream_t st);
+
+// m2: after the planes (its mean among them), the squared deviations from that mean into m2.
+// Under the tile strategy the rows already lie bucketed in the workspace, so that pass is a
+// second tile pass over them: the columns are not read again (20M rows of three float64
+// columns: a scan of 126 us and the other kernels of a call of its own; count, sum, min, max
+// and std of 20M float64 rows into 1023 x 767 720 us a call with that call, 502 without).
+// Under the window strategy it is the scan and spill again (run_window_m2).
+// skip: a record under whose tile strategy the call's window kernels do nothing.
 template <typename TC, typename TV, bool HAS_VAL, int KEYB, bool SQDEV>
 static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &P,
-                      const Planes &out, const double *mean, uint8_t *ws, hipStream_t st) {
+                      const Planes &out, const double *mean, uint8_t *ws, hipStream_t st,
+                      double *m2 = nullptr, const int32_t *skip = nullptr) {
     // Every kernel of this call reads the window from the call's own workspace: a stored
     // window (d->window) is copied in first, so that calls on other streams that share
     // the store and rewrite it cannot hand one call's kernels two different windows.
@@ -2074,10 +2107,10 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     int s;
     if (P.whole) {
         hipLaunchKernelGGL(set_window_kernel, dim3(1), dim3(64), 0, st, window, 0, 0, a.W, a.H,
-                           (int32_t)DSX_STRATEGY_WINDOW);
+                           (int32_t)DSX_STRATEGY_WINDOW, skip);
     } else if (!P.run_window) {  // the tile strategy, forced: no window
         hipLaunchKernelGGL(set_window_kernel, dim3(1), dim3(64), 0, st, window, 0, 0, 0, 0,
-                           (int32_t)DSX_STRATEGY_TILES);
+                           (int32_t)DSX_STRATEGY_TILES, (const int32_t *)nullptr);
     } else if (d->window && d->reuse_window) {
         // the caller's stored record (its window sanitised by every kernel that reads it;
         // its strategy kept only when this call launches both)
@@ -2087,10 +2120,10 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     } else {
         if ((s = fill_async(hist_sel, DSX_FILL_ZERO32, kSelBins, st))) return s;
         hipLaunchKernelGGL((select_hist_kernel<TC>), dim3(64), dim3(1024), 0, st, a, P.bshift,
-                           P.cw, P.ch, hist_sel);
+                           P.cw, P.ch, hist_sel, skip);
         hipLaunchKernelGGL(select_pick_kernel, dim3(1), dim3(1024), 0, st, (const uint32_t *)hist_sel,
                            P.bshift, P.cw, P.ch, a.W, a.H, (int64_t)(P.wl.cap / (uint32_t)ncat),
-                           P.run_tiles ? 1 : 0, window);
+                           P.run_tiles ? 1 : 0, window, skip);
         if (d->window)
             hipLaunchKernelGGL(copy_window_kernel, dim3(1), dim3(64), 0, st,
                                (const int32_t *)window, d->window, 0);
@@ -2214,6 +2247,7 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     pa.max_parts = P.max_parts;
     pa.scratch = ws + P.o_scratch;
     pa.rec = window;
+    pa.window_only = skip ? 1 : 0;
     pa.min_part_tiles = P.tiles_ok ? P.min_part_tiles : (uint32_t)kMinPart;
     unsigned long long *totals = reinterpret_cast<unsigned long long *>(ws + P.o_totals);
     hipLaunchKernelGGL(spill_colscan_kernel, dim3(P.ntiles), dim3(kPartThreads), 0, st, pa, totals);
@@ -2256,8 +2290,67 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
                             (int)P.tile_lds);
     if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
     hipLaunchKernelGGL(merge, dim3(P.ntiles), dim3(kTileThreads), P.tile_lds, st, pa, P.tl,
-                       (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, out);
-    return launch_status();
+                       (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, out,
+                       skip ? (int32_t)DSX_STRATEGY_WINDOW : 0);
+    if ((s = launch_status()) || !m2) return s;
+    if constexpr (HAS_VAL && !SQDEV) {
+        if (P.run_tiles) {  // the same buckets again, one plane (so a smaller region)
+            const Lay L2 = make_lay(PL_SUM, KEYB, P.tl.cap);
+            Planes out2;
+            memset(&out2, 0, sizeof out2);
+            out2.sum = m2;
+            const size_t lds = P.btile_lds - P.tl.bytes + L2.bytes;
+            auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true>;
+            e = hipFuncSetAttribute((const void *)btile, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
+            hipLaunchKernelGGL(btile, dim3(P.max_parts), dim3(kTileThreads), lds, st, pa, ba, L2,
+                               (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells,
+                               (const double *)out.mean, out2);
+            hipLaunchKernelGGL(merge, dim3(P.ntiles), dim3(kTileThreads), (size_t)L2.bytes, st, pa, L2,
+                               (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, out2,
+                               (int32_t)DSX_STRATEGY_TILES);
+            if ((s = launch_status())) return s;
+        }
+        if (P.run_window) return run_window_m2<TC, TV, KEYB>(d, a, P, out.mean, m2, ws, st);
+    }
+    return DSX_OK;
+}
+
+// The m2 pass where the first one may have run the window strategy: a call of its own (one
+// plane, so a larger window, picked for it), whose kernels do nothing where the first pass
+// ran the tile strategy after all (P1.run_tiles: it could).
+// Its workspace starts behind the first pass's record, whose other contents are spent.
+constexpr size_t kM2Base = 256;
+static int m2_plan(const dsx_points_desc *d, const dsx_view *v, const Plan &P1, double *m2,
+                   dsx_points_desc &d2, Plan &P2) {
+    d2 = *d;
+    d2.window = nullptr;
+    d2.reuse_window = 0;
+    // (one plane's tiles may fit the tile strategy where the first pass's did not, and the
+    // strategy passed with a stored window is the first pass's)
+    d2.strategy = P1.run_tiles ? (int32_t)DSX_STRATEGY_WINDOW
+                               : P1.tiles_ok ? d->strategy : (int32_t)DSX_STRATEGY_AUTO;
+    dsx_planes p2;
+    memset(&p2, 0, sizeof p2);
+    p2.sum = m2;
+    return make_plan(&d2, v, &p2, P2);
+}
+template <typename TC, typename TV, int KEYB>
+static int run_window_m2(const dsx_points_desc *d, const PointArgs &a, const Plan &P1, const double *mean,
+                         double *m2, uint8_t *ws, hipStream_t st) {
+    dsx_view v;  // (the plan reads the canvas only)
+    memset(&v, 0, sizeof v);
+    v.width = a.W;
+    v.height = a.H;
+    dsx_points_desc d2;
+    Plan P2;
+    const int s = m2_plan(d, &v, P1, m2, d2, P2);
+    if (s) return s;
+    Planes out2;
+    memset(&out2, 0, sizeof out2);
+    out2.sum = m2;
+    return run_points<TC, TV, true, KEYB, true>(&d2, a, P2, out2, mean, ws + kM2Base, st, nullptr,
+                                                P1.run_tiles ? reinterpret_cast<const int32_t *>(ws) : nullptr);
 }
 
 // ---- canvases beyond the tiles: one pass of global atomics ------------------------------
@@ -2340,14 +2433,15 @@ static int run_global(const dsx_points_desc *d, const PointArgs &a, const dsx_pl
 
 template <typename TC>
 static int dispatch_val(const dsx_points_desc *d, const PointArgs &a, const Plan &P,
-                        const Planes &out, const double *mean, uint8_t *ws, hipStream_t st) {
+                        const Planes &out, const double *mean, uint8_t *ws, hipStream_t st,
+                        double *m2) {
     const bool sq = mean != nullptr;
     if (!has_value(d)) return run_points<TC, float, false, 8, false>(d, a, P, out, mean, ws, st);
     if (d->val_dtype == DSX_F32)
         return sq ? run_points<TC, float, true, 4, true>(d, a, P, out, mean, ws, st)
-                  : run_points<TC, float, true, 4, false>(d, a, P, out, mean, ws, st);
+                  : run_points<TC, float, true, 4, false>(d, a, P, out, mean, ws, st, m2);
     return sq ? run_points<TC, double, true, 8, true>(d, a, P, out, mean, ws, st)
-              : run_points<TC, double, true, 8, false>(d, a, P, out, mean, ws, st);
+              : run_points<TC, double, true, 8, false>(d, a, P, out, mean, ws, st, m2);
 }
 
 // ---- indexed aggregation (rows sorted by the cells of a lattice) ------------------------
@@ -2685,9 +2779,30 @@ extern "C" size_t dsx_points_workspace_size(const dsx_points_desc *d, const dsx_
     return P.total;
 }
 
-extern "C" int dsx_points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
-                              const double *mean, void *workspace, size_t workspace_bytes,
-                              void *stream) {
+// The workspace of a call with an m2 plane: its two passes share it.
+static int m2_total(const dsx_points_desc *d, const dsx_view *v, const Plan &P, double *m2, size_t &total) {
+    total = P.total;
+    if (P.global || !P.run_window) return DSX_OK;
+    dsx_points_desc d2;
+    Plan P2;
+    const int st = m2_plan(d, v, P, m2, d2, P2);
+    if (st) return st;
+    if (kM2Base + P2.total > total) total = kM2Base + P2.total;
+    return DSX_OK;
+}
+
+extern "C" size_t dsx_points_m2_workspace_size(const dsx_points_desc *d, const dsx_view *v,
+                                               const dsx_planes *p) {
+    if (check_points(d, v) || !p || !p->mean || !has_value(d)) return 0;
+    Plan P;
+    size_t total;
+    if (make_plan(d, v, p, P) || m2_total(d, v, P, p->mean, total)) return 0;
+    return total;
+}
+
+static int points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
+                      const double *mean, double *m2, void *workspace, size_t workspace_bytes,
+                      void *stream) {
     int st = check_points(d, v);
     if (st) return st;
     if (!p) return DSX_ERR_NULL;
@@ -2698,18 +2813,39 @@ extern "C" int dsx_points_agg(const dsx_points_desc *d, const dsx_view *v, const
     if (p->mean && !has_value(d)) return DSX_ERR_ACCUM;
     Plan P;
     if ((st = make_plan(d, v, p, P))) return st;
+    size_t total = P.total;
+    if (m2 && (st = m2_total(d, v, P, m2, total))) return st;
     if (!workspace) return DSX_ERR_WORKSPACE;
-    if (workspace_bytes < P.total) return DSX_ERR_WORKSPACE;
+    if (workspace_bytes < total) return DSX_ERR_WORKSPACE;
     const PointArgs a = args_of(d, v);
     const Planes out = planes_of(p);
     hipStream_t s = as_stream(stream);
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     if (P.global) {
-        if (d->xy_dtype == DSX_F32) return run_global<float>(d, a, p, out, mean, ws, s);
-        return run_global<double>(d, a, p, out, mean, ws, s);
+        dsx_planes p2;
+        memset(&p2, 0, sizeof p2);
+        p2.sum = m2;
+        const bool f32 = d->xy_dtype == DSX_F32;
+        st = f32 ? run_global<float>(d, a, p, out, mean, ws, s) : run_global<double>(d, a, p, out, mean, ws, s);
+        if (st || !m2) return st;
+        return f32 ? run_global<float>(d, a, &p2, planes_of(&p2), p->mean, ws, s)
+                   : run_global<double>(d, a, &p2, planes_of(&p2), p->mean, ws, s);
     }
-    if (d->xy_dtype == DSX_F32) return dispatch_val<float>(d, a, P, out, mean, ws, s);
-    return dispatch_val<double>(d, a, P, out, mean, ws, s);
+    if (d->xy_dtype == DSX_F32) return dispatch_val<float>(d, a, P, out, mean, ws, s, m2);
+    return dispatch_val<double>(d, a, P, out, mean, ws, s, m2);
+}
+
+extern "C" int dsx_points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
+                              const double *mean, void *workspace, size_t workspace_bytes,
+                              void *stream) {
+    return points_agg(d, v, p, mean, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsx_points_agg_m2(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
+                                 double *m2, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!p || !m2) return DSX_ERR_NULL;
+    if (!p->mean) return DSX_ERR_ACCUM;
+    return points_agg(d, v, p, nullptr, m2, workspace, workspace_bytes, stream);
 }
 
 // ---- row-index reductions ---------------------------------------------------------------
@@ -3178,10 +3314,11 @@ static int riw_launch(const dsx_points_desc *d, const RiwArgs &r, const RiwPlan 
     } else {
         if ((s = fill_async(hist_sel, DSX_FILL_ZERO32, kSelBins, st))) return s;
         hipLaunchKernelGGL((select_hist_kernel<TC>), dim3(64), dim3(1024), 0, st, r.a, P.bshift,
-                           P.cw, P.ch, hist_sel);
+                           P.cw, P.ch, hist_sel, (const int32_t *)nullptr);
         hipLaunchKernelGGL(select_pick_kernel, dim3(1), dim3(1024), 0, st,
                            (const uint32_t *)hist_sel, P.bshift, P.cw, P.ch, r.a.W, r.a.H,
-                           (int64_t)(P.cap / (uint32_t)r.a.cat.ncat), 0, window);
+                           (int64_t)(P.cap / (uint32_t)r.a.cat.ncat), 0, window,
+                           (const int32_t *)nullptr);
         if (d->window)
             hipLaunchKernelGGL(copy_window_kernel, dim3(1), dim3(64), 0, st,
                                (const int32_t *)window, d->window, 0);

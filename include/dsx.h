@@ -167,6 +167,16 @@ size_t dsx_points_workspace_size(const dsx_points_desc *d, const dsx_view *v,
 int dsx_points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
                    const double *mean, void *workspace, size_t workspace_bytes, void *stream);
 
+/* The planes of dsx_points_agg, a finalized mean among them, and the m2 of var / std in one
+ * call: m2 (a device f64 plane of H*W*ncat cells) receives sum((v - mean[bin])^2).  Same
+ * results as dsx_points_agg followed by dsx_points_agg with mean; the rows that the first
+ * pass bucketed by tile are not read from the columns again.  Needs a workspace of
+ * dsx_points_m2_workspace_size bytes. */
+size_t dsx_points_m2_workspace_size(const dsx_points_desc *d, const dsx_view *v,
+                                    const dsx_planes *p);
+int dsx_points_agg_m2(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p, double *m2,
+                      void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- lines ---------------------------------------------------------------------- *
  * nlines lines of nverts vertices each.  Vertex k of line l is
  *   x = X[l*x_line_stride + k*x_vert_stride],  y = Y[l*y_line_stride + k*y_vert_stride]
