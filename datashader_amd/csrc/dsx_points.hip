@@ -1950,6 +1950,21 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     while (P.tshift > kMinTileShift && ((P.ncells + (1ll << P.tshift) - 1) >> P.tshift) < cus)
         --P.tshift;
     while ((P.ncells + (1ll << P.tshift) - 1) >> P.tshift > kMaxTiles) ++P.tshift;
+    // tiles of twice the size (one workgroup a CU) where only their buckets fit the tile
+    // strategy's scan: without it every row of data spread over the canvas is spilled
+    // (count, sum, min, max, std of 20M float64 rows into 1800 x 1000: 847 us a call with
+    // 2048-cell tiles, 434 with 4096).  The strategy asked for has no say: the window's
+    // size follows from the tiles, and a stored window is used again under either.
+    {
+        const size_t vb = (size_t)P.vbytes;
+        const auto fits = [&](int sh) {
+            const size_t nb = (size_t)((P.ncells + (1ll << sh) - 1) >> sh);
+            return bkt_layout(vb, nb, (size_t)kBktMinC, P) <= (size_t)kLdsBytes - 512;
+        };
+        const int64_t ids = 4 * (kBktBatch + 2 * (int64_t)cus + 1);
+        if (!fits(P.tshift) && fits(P.tshift + 1) && (2ll << P.tshift) * cb + 16 + ids <= kLdsBytes)
+            ++P.tshift;
+    }
     const int64_t tcap = 1ll << P.tshift;
     P.global = false;
     if (tcap * (int64_t)cb > kLdsBytes - 16) {
