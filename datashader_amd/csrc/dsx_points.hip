@@ -1166,6 +1166,11 @@ __device__ void tile_store(const uint8_t *smem, const Lay &L, const PartArgs &p,
     const Window w = load_window(window, W, H, wcap_px);
     int64_t c1 = c0 + p.tile_cells;
     if (c1 > ncells) c1 = ncells;
+    if (w.w == 0 || w.h == 0) {  // uniform: no window, no divisions for the cell's pixel
+        for (uint32_t c = threadIdx.x; c < (uint32_t)(c1 - c0); c += kTileThreads)
+            region_store<KEYB>(smem, L, c, out, c0 + c);
+        return;
+    }
     for (int64_t gcell = c0 + threadIdx.x; gcell < c1; gcell += kTileThreads) {
         // cells < 2^32 (checked on the host): 32-bit divisions, not 64-bit ones
         const uint32_t gc = (uint32_t)gcell;
@@ -1360,6 +1365,7 @@ struct BktArgs {
     uint32_t o_cnt, o_lo, o_tblk, o_base, o_bk, o_fl, o_off, o_val, o_ctrl;  // scan LDS offsets
     uint32_t loc_cap;              // block indices the bucket area of LDS holds
     uint32_t batch;                // block ids the tile pass stages at a time
+    uint32_t o_mean;               // the tile pass's LDS offset of the tile's means
 };
 
 // The tile strategy's scan.  Bucket b's slots are numbered from its LDS block: slots
@@ -1746,7 +1752,7 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
 // four times the bytes are in flight per load instruction.
 template <typename TV, bool HAS_VAL>
 struct BktRows {
-    static constexpr int kU = 4;
+    static constexpr int kU = sizeof(TV) == 8 ? 2 : 4;  // (float64 values: 71 us with 4, 65 with 2)
     uint2 o[kU];
     TV v[kU][4];
 
@@ -1771,7 +1777,12 @@ struct BktRows {
 
 // The tile strategy's tile pass: part `blockIdx.x` of tile t aggregates its share of
 // the tile's blocks in LDS (a split tile leaves its planes to tile_merge_kernel).
-template <typename TV, bool HAS_VAL, int KEYB, bool SQDEV>
+// MLDS (with SQDEV): the tile's means lie in LDS, copied there first: read from global
+// memory row by row, each read also waited for the rows loaded ahead (20M float64 rows into
+// 1023 x 767: 92 us, 50 from LDS).  WF: the plane set when known at compile time (0: read
+// from the layout).  What is left is the reads of scattered blocks (without the updates
+// 50M float32 rows take 80 of 84 us) and the two rounds of workgroups of ~700 tiles.
+template <typename TV, bool HAS_VAL, int KEYB, bool SQDEV, bool MLDS = false, uint32_t WF = 0>
 __global__ __launch_bounds__(kTileThreads) void btile_agg_kernel(PartArgs p, BktArgs s, Lay L,
                                                                 const int32_t *window, int32_t W,
                                                                 int32_t H, int64_t wcap_px,
@@ -1804,6 +1815,12 @@ __global__ __launch_bounds__(kTileThreads) void btile_agg_kernel(PartArgs p, Bkt
         ex[g] = g < G ? p.hist[(size_t)g * p.ntiles + t] : (uint32_t)(te - tb);
         if (g < G) lpg[g] = s.lpre[(size_t)g * s.nb + t];
     }
+    const double *lmean = reinterpret_cast<const double *>(smem + s.o_mean);  // [L.cap]
+    if constexpr (MLDS) {
+        double *lm = reinterpret_cast<double *>(smem + s.o_mean);
+        for (uint32_t c = threadIdx.x; c < L.cap; c += kTileThreads)
+            lm[c] = c0 + (int64_t)c < ncells ? mean[c0 + c] : 0.0;
+    }
     for (unsigned long long bb = b; bb < e; bb += s.batch) {
         const uint32_t nbb = (uint32_t)(e - bb < (unsigned long long)s.batch ? e - bb : s.batch);
         __syncthreads();  // the region and ex / lpg are written, the last batch's ids are read
@@ -1828,39 +1845,52 @@ __global__ __launch_bounds__(kTileThreads) void btile_agg_kernel(PartArgs p, Bkt
         }
         __syncthreads();
         const uint32_t ngrp = nbb << (s.cshift - 2u);  // groups of four entries
-        R ra, rb, rc;  // three register sets rotate roles, as in the scan
+        // three register sets rotate roles, as in the scan; with values two (the registers
+        // of the third cost more than its loads in flight gave: the statistics tiles of 20M
+        // float64 rows 87 us with three, 71 with two)
+        constexpr bool kTwo = HAS_VAL;
+        R ra, rb, rc;
         ra.load(s, sblk, 0u, ngrp);
-        rb.load(s, sblk, kStep, ngrp);
+        if constexpr (!kTwo) rb.load(s, sblk, kStep, ngrp);
         uint32_t g0 = 0u;
         auto step = [&](R &cur, R &far) {
-            far.load(s, sblk, g0 + 2u * kStep, ngrp);
+            far.load(s, sblk, g0 + (kTwo ? kStep : 2u * kStep), ngrp);
 #pragma unroll
             for (int u = 0; u < R::kU; ++u) {
-                if (g0 + (uint32_t)(u * kTileThreads + threadIdx.x) >= ngrp) continue;
+                const bool in = g0 + (uint32_t)(u * kTileThreads + threadIdx.x) < ngrp;
+                // the four rows' means are read together, before the first update
+                uint32_t lc[4];
+                double add[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint32_t lc = ((e < 2 ? cur.o[u].x : cur.o[u].y) >> (16 * (e & 1))) & 0xFFFFu;
-                    if (lc >= L.cap) continue;  // an unused slot of a partial block
-                    double v = 0.0;
-                    bool vnan = true;
-                    if constexpr (HAS_VAL) {
-                        v = (double)cur.v[u][e];
-                        vnan = v != v;
-                    }
-                    double add = v;
+                    lc[e] = ((e < 2 ? cur.o[u].x : cur.o[u].y) >> (16 * (e & 1))) & 0xFFFFu;
+                    if (!in) lc[e] = kBktUnused;
+                    add[e] = HAS_VAL ? (double)cur.v[u][e] : 0.0;
                     if constexpr (SQDEV) {
-                        const double d = v - mean[c0 + lc];
-                        add = d * d;
+                        const double m = MLDS ? lmean[lc[e] < L.cap ? lc[e] : 0u]
+                                              : lc[e] < L.cap ? mean[c0 + lc[e]] : 0.0;
+                        const double d = add[e] - m;
+                        add[e] = d * d;
                     }
-                    region_add<KEYB>(smem, L, lc, vnan, v, add);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (lc[e] >= L.cap) continue;  // past the batch, or an unused slot of a partial block
+                    const double v = HAS_VAL ? (double)cur.v[u][e] : 0.0;
+                    region_add<KEYB, WF>(smem, L, lc[e], !HAS_VAL || v != v, v, add[e]);
                 }
             }
             g0 += kStep;
         };
         while (g0 < ngrp) {  // steps past ngrp load group 0 and add nothing
-            step(ra, rc);
-            step(rb, ra);
-            step(rc, rb);
+            if constexpr (kTwo) {
+                step(ra, rb);
+                step(rb, ra);
+            } else {
+                step(ra, rc);
+                step(rb, ra);
+                step(rc, rb);
+            }
         }
     }
     __syncthreads();
@@ -2219,6 +2249,7 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
         ba.o_ctrl = P.bo_ctrl;
         ba.loc_cap = P.bo_cnt / 4u;  // values and offsets come first, from byte 0
         ba.batch = P.batch;
+        ba.o_mean = 0;
         auto bscan = bscan_kernel<TC, TV, HAS_VAL, CK_ANY, false>;
         if (ck == CK_NONE)
             bscan = lin ? bscan_kernel<TC, TV, HAS_VAL, CK_NONE, true>
@@ -2291,7 +2322,10 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
         if ((s = launch_status())) return s;
     }
     if (P.run_tiles) {
-        auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV>;
+        // (a squared-deviation pass has the sum plane only, one without values the count only)
+        constexpr uint32_t kOne = SQDEV ? PL_SUM : HAS_VAL ? 0u : PL_CNT;
+        auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, false, kOne>;
+        if (P.tl.flags != kOne) btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV>;
         e = hipFuncSetAttribute((const void *)btile, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)P.btile_lds);
         if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
@@ -2314,8 +2348,15 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
             Planes out2;
             memset(&out2, 0, sizeof out2);
             out2.sum = m2;
-            const size_t lds = P.btile_lds - P.tl.bytes + L2.bytes;
-            auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true>;
+            size_t lds = P.btile_lds - P.tl.bytes + L2.bytes;
+            auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true, false, PL_SUM>;
+            // the tile's means in LDS too where two workgroups still fit a CU
+            const size_t o_mean = align_up(lds, 16), with = o_mean + 8 * (size_t)P.tl.cap;
+            if (with <= (size_t)kLdsBytes / 2) {
+                btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true, true, PL_SUM>;
+                ba.o_mean = (uint32_t)o_mean;
+                lds = with;
+            }
             e = hipFuncSetAttribute((const void *)btile, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
             hipLaunchKernelGGL(btile, dim3(P.max_parts), dim3(kTileThreads), lds, st, pa, ba, L2,

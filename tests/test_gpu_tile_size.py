@@ -55,3 +55,29 @@ def test_planes(strategy, spread, dt, W, H):
                     np.testing.assert_array_equal(got["c"].values, cf.count(b, W, H))
     finally:
         backend.FORCE_STRATEGY = None
+
+
+@pytest.mark.parametrize("W,H", [(1000, 700), (2600, 1500)], ids=["means-in-lds", "means-gathered"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_std_over_tiles(dt, W, H):
+    """The second tile pass with its tile's means in LDS, and where they do not fit there."""
+    n = 300_001
+    rng = np.random.default_rng(H)
+    x, y = rng.random((2, n)).astype(dt)
+    v = rng.normal(100, 3, n).astype(dt)
+    v[::17] = np.nan
+    f = dsa.DeviceFrame({k: torch.from_numpy(a).cuda() for k, a in (("x", x), ("y", y), ("v", v))})
+    cvs = dsa.Canvas(W, H, x_range=(0.0, 1.0), y_range=(0.0, 1.0))
+    b = cf.point_bins(x, y, G.view_for(W, H, (0.0, 1.0), (0.0, 1.0)), W, H)
+    backend.FORCE_STRATEGY = _abi.STRATEGY_TILES
+    try:
+        got = cvs.points(f, "x", "y", dsa.summary(m=dsa.mean("v"), s=dsa.std("v")))
+        torch.cuda.synchronize()
+    finally:
+        backend.FORCE_STRATEGY = None
+    want = np.sqrt(cf.var2pass(b, v, W, H))
+    ok = ~np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got["s"].values), ~ok)
+    # (as for std elsewhere: 1e-9 for float64 values, 1e-5 for float32)
+    np.testing.assert_allclose(got["s"].values[ok], want[ok], rtol=1e-5 if dt is np.float32 else 1e-9, atol=1e-9)
+    np.testing.assert_allclose(got["m"].values, cf.mean(b, v, W, H), rtol=1e-12)
