@@ -13,7 +13,7 @@ from __future__ import annotations
 import numpy as np
 import pandas as pd
 
-from . import _abi
+from . import _abi, _upload
 
 _KIND = {np.dtype("float32"): "f4", np.dtype("float64"): "f8", np.dtype("int8"): "i1",
          np.dtype("int16"): "i2", np.dtype("int32"): "i4", np.dtype("int64"): "i8",
@@ -135,6 +135,10 @@ def _torch_kind(t):
     return m.get(t.dtype, "O")
 
 
+def _torch_dtype(dt):
+    return _torch().from_numpy(np.empty(0, dtype=dt)).dtype
+
+
 class DeviceFrame:
     """Columns resident in device memory.
 
@@ -160,11 +164,11 @@ class DeviceFrame:
         torch = _torch()
         cols, cats = {}, {}
         groups = {}
+        plain = {}
         for name in df.columns:
             dt = df.dtypes[name]
             if isinstance(dt, pd.CategoricalDtype):
-                codes = np.ascontiguousarray(df[name].cat.codes.to_numpy())
-                cols[name] = torch.from_numpy(codes).to(device)
+                plain[name] = df[name].cat.codes.to_numpy()
                 cats[name] = list(dt.categories)
             elif is_ragged(df[name]):
                 cols[name] = RaggedColumn.from_series(df[name], device)
@@ -173,16 +177,32 @@ class DeviceFrame:
             elif np.dtype(dt).kind == "f":
                 groups.setdefault(np.dtype(dt), []).append(name)
             elif np.dtype(dt).kind in "iub":
-                cols[name] = torch.from_numpy(np.ascontiguousarray(df[name].to_numpy())).to(device)
+                plain[name] = df[name].to_numpy()
             else:
                 continue  # non-numeric columns stay on the host (never aggregated)
-        for dt, names in groups.items():
-            host = np.empty((len(names), len(df)), dtype=dt)
-            for j, name in enumerate(names):
-                host[j] = df[name].to_numpy()
-            block = torch.from_numpy(host).to(device)
-            for j, name in enumerate(names):
-                cols[name] = block[j]
+        floats = {name: df[name].to_numpy() for names in groups.values() for name in names}
+        nbytes = sum(a.nbytes for a in (*plain.values(), *floats.values()))
+        if torch.device(device).type == "cuda" and nbytes >= _upload.MIN_BYTES:
+            pairs = []
+            for name, a in plain.items():
+                cols[name] = torch.empty(len(df), dtype=_torch_dtype(a.dtype), device=device)
+                pairs.append((a, cols[name]))
+            for dt, names in groups.items():
+                block = torch.empty((len(names), len(df)), dtype=_torch_dtype(dt), device=device)
+                for j, name in enumerate(names):
+                    cols[name] = block[j]
+                    pairs.append((floats[name], block[j]))
+            _upload.upload(pairs)
+        else:
+            for name, a in plain.items():
+                cols[name] = torch.from_numpy(np.ascontiguousarray(a)).to(device)
+            for dt, names in groups.items():
+                host = np.empty((len(names), len(df)), dtype=dt)
+                for j, name in enumerate(names):
+                    host[j] = floats[name]
+                block = torch.from_numpy(host).to(device)
+                for j, name in enumerate(names):
+                    cols[name] = block[j]
         ordered = {name: cols[name] for name in df.columns if name in cols}
         return cls(ordered, cats)
 
