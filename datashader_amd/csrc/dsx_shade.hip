@@ -591,7 +591,10 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(int64_t n, Ws w, in
     part_init(p);
     for_pixels(n, [&](int64_t i) { return plane.load(i); }, [&](int64_t i, auto raw) {
         const double x = plane.value(raw, P);
-        if (x != x) { w.val[i] = x; return; }
+        if (x != x) {
+            if constexpr (Plane::kRaw) w.val[i] = x;  // (a working plane holds it already)
+            return;
+        }
         double t;
         if (how == DSX_HOW_EQ_HIST) {
             if (P.int_path) {
