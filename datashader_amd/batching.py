@@ -91,7 +91,7 @@ class BatchEngine:
         c.cell_start = dev.ptr(index.frame.grid_index["cell_start"])
         c.max_requests, c.max_tiles, c.max_regions = max_requests, max_tiles, max_regions
         c.threads = threads
-        c.workgroups = workgroups or _device_count() * (1024 // threads)
+        c.workgroups = workgroups or _device_count()
         self.max_requests, self.max_tiles = max_requests, max_tiles
         ws = int(lib.dsx_batch_workspace_size(c))
         if ws == 0:
@@ -175,13 +175,6 @@ class Tuning:
     large tiles."""
 
     DEFAULT = {"tile_h": 64, "tile_cells": 0, "part_rows": 1 << 18}
-    # views of more rows per cell than this, densest first: (rows per cell, knobs).  Small
-    # tiles are held several times over in LDS, which dense views need (their rows meet in
-    # few pixels); a sparse view's small tiles would each re-read the lattice cells they
-    # share.  24 viewports over 100M rows, aggregation kernel: 2.36 ms with the default for
-    # all, 1.69 with these, 1.95 with tiles of 512, 1.84 with 2048.
-    DENSE = ((16.0, {"tile_h": 32, "tile_cells": 1024, "part_rows": 1 << 18}),
-             (2.0, {"tile_h": 64, "tile_cells": 4096, "part_rows": 1 << 18}))
 
     def __init__(self, threads=1024, workgroups=None, per_class=None):
         self.threads, self.workgroups = threads, workgroups
@@ -195,12 +188,7 @@ class Tuning:
         return (int(np.log2(cells)), dc)
 
     def knobs(self, W, H, rows):
-        tuned = self.per_class.get(self.key(W, H, rows))
-        if tuned is not None:
-            return tuned
-        if "DEFAULT" in self.__dict__:  # set on this tuning: for every class not tuned
-            return self.DEFAULT
-        return next((k for d, k in self.DENSE if rows >= d * W * H), self.DEFAULT)
+        return self.per_class.get(self.key(W, H, rows), self.DEFAULT)
 
     def to_dict(self):
         return {"threads": self.threads, "workgroups": self.workgroups,

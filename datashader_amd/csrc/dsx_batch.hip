@@ -37,9 +37,8 @@
 namespace dsx {
 
 constexpr int kBLds = 160 * 1024;
-constexpr int kBMaxGrid = 4096;               // cells a side of the largest lattice
-constexpr int kBTableRows = 256;              // lattice rows tabled in LDS at a time
-constexpr int kBTable = kBTableRows * 8;      // LDS: first row + row prefix (u32) per lattice row
+constexpr int kBMaxLatRows = 4096;            // lattice rows a tile may span: the largest grid
+constexpr int kBTable = kBMaxLatRows * 8;     // LDS: first row + row prefix (u32) per lattice row
 constexpr int kBTileThreads = 256;
 constexpr int kBItemThreads = 1024;
 constexpr int kBHeader = 256;                 // bytes of the table header
@@ -317,8 +316,8 @@ __global__ __launch_bounds__(kBItemThreads) void b_items_kernel(BArgs A) {
 }
 
 // ---- agg: persistent workgroups over the work queue ---------------------------------
-__device__ __forceinline__ void b_region_init(uint8_t *r, const BLay &L, uint32_t used, int tid, int nt) {
-    for (uint32_t c = tid; c < used; c += nt) {
+__device__ __forceinline__ void b_region_init(uint8_t *r, const BLay &L, int tid, int nt) {
+    for (uint32_t c = tid; c < L.cap; c += nt) {
         reinterpret_cast<uint32_t *>(r + L.o_cnt)[c] = 0u;
         if (L.has_val) {
             reinterpret_cast<double *>(r + L.o_sum)[c] = 0.0;
@@ -327,371 +326,249 @@ __device__ __forceinline__ void b_region_init(uint8_t *r, const BLay &L, uint32_
     }
 }
 
-// Write the output cell g from its rows n, NaN rows nn and sum s: the finalizers of
+// Write cell c of a finished region as the tile's output cell g: the finalizers of
 // count(), count(v), sum(v) (NaN where no value) and mean(v).
-__device__ __forceinline__ void b_store_values(const BReq &q, int64_t g, bool has_val, uint32_t n,
-                                               uint32_t nn, double s) {
+__device__ __forceinline__ void b_store_cell(const uint8_t *r, const BLay &L, uint32_t c,
+                                             const BReq &q, int64_t g) {
+    const uint32_t n = reinterpret_cast<const uint32_t *>(r + L.o_cnt)[c];
     if (q.count) global_ptr(q.count)[g] = n;
-    if (!has_val) return;
-    const uint32_t nv = n - nn;
+    if (!L.has_val) return;
+    const uint32_t nv = n - reinterpret_cast<const uint32_t *>(r + L.o_nan)[c];
+    const double s = reinterpret_cast<const double *>(r + L.o_sum)[c];
     if (q.countv) global_ptr(q.countv)[g] = nv;
     if (q.sum) global_ptr(q.sum)[g] = nv > 0u ? s : (double)NAN;
     if (q.mean) global_ptr(q.mean)[g] = nv > 0u ? s / (double)nv : (double)NAN;
 }
 
-// Copies of a tile's cells in the LDS region, as a power of two: a small tile is held
-// several times over, cell c's copies side by side (other banks), and each lane adds to
-// its own: the rows of a dense view are sorted by lattice cell, so the lanes of a wave
-// meet in a few pixels, and LDS atomics to one address run one after the other.  (24
-// viewports over 100M rows: atomics 1.0 of 2.4 ms of the kernel with one copy.)
-constexpr uint32_t kBMaxCopies = 3;  // log2: eight
-__device__ __forceinline__ uint32_t b_copies(const BLay &L, const BReq &q) {
-    uint32_t cl = 0;
-    while (cl < kBMaxCopies && ((uint32_t)(q.tw * q.th) << (cl + 1)) <= L.cap) ++cl;
-    return cl;
-}
-
-// Cell c of a region: its copies' rows, NaN rows and sum.
-__device__ __forceinline__ void b_fold_cell(const uint8_t *r, const BLay &L, uint32_t c, uint32_t cl,
-                                            uint32_t &n, uint32_t &nn, double &s) {
-    n = nn = 0;
-    s = 0.0;
-    for (uint32_t i = c << cl; i < (c + 1) << cl; ++i) {
-        n += reinterpret_cast<const uint32_t *>(r + L.o_cnt)[i];
-        if (L.has_val) {
-            nn += reinterpret_cast<const uint32_t *>(r + L.o_nan)[i];
-            s += reinterpret_cast<const double *>(r + L.o_sum)[i];
-        }
-    }
-}
-
-__device__ __forceinline__ void b_store_tile(const uint8_t *r, const BLay &L, uint32_t cl,
-                                             const BReq &q, int32_t t, int nt) {
+__device__ __forceinline__ void b_store_tile(const uint8_t *r, const BLay &L, const BReq &q,
+                                             int32_t t, int nt) {
     int32_t px0, px1, py0, py1;
     b_tile_rect(q, t, px0, px1, py0, py1);
     const int32_t w = px1 - px0, h = py1 - py0;
     for (int32_t c = threadIdx.x; c < w * h; c += nt) {
         const int32_t ly = c / w, lx = c - ly * w;
-        uint32_t n, nn;
-        double s;
-        b_fold_cell(r, L, (uint32_t)(ly * q.tw + lx), cl, n, nn, s);
-        b_store_values(q, (int64_t)(py0 + ly) * q.W + (px0 + lx), L.has_val, n, nn, s);
+        b_store_cell(r, L, (uint32_t)(ly * q.tw + lx), q, (int64_t)(py0 + ly) * q.W + (px0 + lx));
     }
 }
 
-// Four consecutive rows of a column, at any row (a 16-byte load needs 4-byte alignment).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int kBItems = 4;  // rows per thread per iteration, loads issued together
 
-constexpr int kBStep = 256;  // rows a wave takes at a time: four consecutive ones a lane
-
-// One step of a wave: rows [row, end) of the sorted set (all of one lattice row, at most
-// kBStep), lane l holding rows row + 4 l .. + 3.
-template <bool VAL>
-struct BRows {
-    uint32_t row, end;   // uniform; row == end: none
-    f32x4 x, y, v;
-
-    // The last readable group starts at row n - 4: a lane past it reads that one and finds
-    // its rows by number (n < 4: row by row).
-    __device__ __forceinline__ uint32_t at(const BArgs &A, int lane) const {
-        const uint32_t r = row + 4u * (uint32_t)lane, last = A.n >= 4 ? (uint32_t)(A.n - 4) : 0u;
-        return r < last ? r : last;
-    }
-    __device__ __forceinline__ static f32x4 read(const float *p, uint32_t at, int64_t n) {
-        if (n >= 4) return *reinterpret_cast<const f32x4_row *>(p + at);
-        f32x4 r = {0.f, 0.f, 0.f, 0.f};
-        for (int e = 0; e < 4; ++e)
-            if (e < n) r[e] = p[e];
-        return r;
-    }
-    __device__ __forceinline__ void load(const BArgs &A, int lane) {
-        const uint32_t a = at(A, lane);
-        x = read(A.x, a, A.n);
-        y = read(A.y, a, A.n);
-        if constexpr (VAL) v = read(A.v, a, A.n);
-    }
-};
-
-// Persistent workgroups pop (tile, part) items until the queue is drained.  A part is a
-// range of the tile's rows, numbered through its lattice rows; each wave takes a
-// contiguous share of it and walks the lattice rows in order (no search per row), 256 rows
-// a step, two steps' loads in flight behind the one that is binned.  The rows are sorted
-// by lattice cell, so in a dense view a lane's four rows, or all 256 of a step, often land
-// in one pixel: they are then added as one.
-// 24 viewports over 100M rows (546M rows read, 6.6 GB, 9209 items): 2.62 ms with a table
-// search per row and one copy of a tile, 2.36 ms without the searches, 1.69 ms with small
-// tiles in up to eight copies; 1.37 ms of it are the loads alone (4.8 TB/s), 0.1-0.2 ms the
-// LDS atomics.  Waves that interleave their steps, two workgroups of 512 threads a CU:
-// the same time.
-template <int NT, bool VAL>
-__global__ __launch_bounds__(NT, 4) void b_agg_kernel(BArgs A) {
+template <int NT>
+__global__ __launch_bounds__(NT) void b_agg_kernel(BArgs A) {
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ uint32_t s_wave[NT / 64];
+    __shared__ unsigned long long sh[NT / 64 + 1];
     __shared__ uint32_t s_item;
     const BLay &L = A.L;
-    // a batch of the tile's lattice rows: first sorted row and row-count prefix (n < 2^32)
+    // the tile's lattice rows: first sorted row and row-count prefix, 32-bit (n < 2^32)
     uint32_t *s_start = reinterpret_cast<uint32_t *>(smem + L.bytes);
-    uint32_t *s_pre = s_start + kBTableRows;
-    uint32_t *const l_cnt = reinterpret_cast<uint32_t *>(smem + L.o_cnt);
-    uint32_t *const l_nan = reinterpret_cast<uint32_t *>(smem + L.o_nan);
-    double *const l_sum = reinterpret_cast<double *>(smem + L.o_sum);
-    const int lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const auto uni = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
-    if (threadIdx.x == 0) s_item = atomicAdd(&A.ctr[0], 1u);
+    uint32_t *s_pre = s_start + kBMaxLatRows;
     for (;;) {
+        if (threadIdx.x == 0) s_item = atomicAdd(&A.ctr[0], 1u);
         __syncthreads();
         const uint32_t item = s_item;
         if (item >= A.ctr[1]) break;   // every workgroup leaves once the queue is drained
-        uint32_t next = 0;             // the next item, popped ahead of its use
-        if (threadIdx.x == 0) next = atomicAdd(&A.ctr[0], 1u);
         const BItem m = A.items[item];
         const BTile d = A.tiles[m.tile];
         const BReq q = A.reqs[d.req];
         int32_t px0, px1, py0, py1;
         b_tile_rect(q, d.t, px0, px1, py0, py1);
-        const uint32_t cl = b_copies(L, q), mine = (uint32_t)lane & ((1u << cl) - 1u);
-        b_region_init(smem, L, (uint32_t)(q.tw * q.th) << cl, threadIdx.x, NT);
-        const uint32_t tw = (uint32_t)(px1 - px0), th = (uint32_t)(py1 - py0);
-        // this part's rows [plo, phi) of the tile's rows (numbered through its lattice rows)
-        const uint64_t rows = d.rows;
-        const uint64_t E = d.nparts > 1 ? (rows + d.nparts - 1) / d.nparts : rows;
-        const uint64_t plo = (uint64_t)m.part * E < rows ? (uint64_t)m.part * E : rows;
-        const uint64_t phi = plo + E < rows ? plo + E : rows;
-        const int32_t nlat = d.gx0 <= d.gx1 ? d.gy1 - d.gy0 + 1 : 0;
-        uint64_t base = 0;  // rows of the tile in the batches before this one
-        for (int32_t k0 = 0; k0 < nlat && base < phi; k0 += kBTableRows) {
-        const int32_t nr = nlat - k0 < kBTableRows ? nlat - k0 : kBTableRows;
-        uint32_t tot;  // rows in this batch
-        {
-            const int32_t k = (int32_t)threadIdx.x;
-            uint32_t len = 0, st0 = 0;
-            if (k < nr) {
-                const int64_t row = (int64_t)(d.gy0 + k0 + k) * A.grid;
-                st0 = (uint32_t)A.cs[row + d.gx0];
-                len = (uint32_t)A.cs[row + d.gx1 + 1] - st0;
+        // lattice rows of the tile (at most the grid's 4096)
+        const int32_t nrow = d.gx0 <= d.gx1 ? d.gy1 - d.gy0 + 1 : 0;
+        unsigned long long tot = 0;
+        for (int32_t k0 = 0; k0 < nrow; k0 += NT) {
+            const int32_t k = k0 + (int32_t)threadIdx.x;
+            unsigned long long len = 0;
+            int64_t st0 = 0;
+            if (k < nrow) {
+                const int64_t row = (int64_t)(d.gy0 + k) * A.grid;
+                st0 = A.cs[row + d.gx0];
+                len = (unsigned long long)(A.cs[row + d.gx1 + 1] - st0);
             }
-            // exclusive scan over the first kBTableRows threads (four waves)
-            uint32_t x = len;
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t y = __shfl_up(x, off, 64);
-                if (lane >= off) x += y;
+            unsigned long long t2;
+            const unsigned long long ex = b_block_exscan(len, sh, t2);
+            if (k < nrow) {
+                s_start[k] = (uint32_t)st0;
+                s_pre[k] = (uint32_t)(tot + ex);
             }
-            if (lane == 63) s_wave[wave] = x;
-            __syncthreads();  // (also: the last batch's table is no longer read)
-            uint32_t before = 0;
-            tot = 0;
-#pragma unroll
-            for (uint32_t w = 0; w < (uint32_t)kBTableRows / 64; ++w) {
-                before += w < wave ? s_wave[w] : 0u;
-                tot += s_wave[w];
-            }
-            if (k < nr) {
-                s_start[k] = st0;
-                s_pre[k] = before + x - len;
-            }
-            __syncthreads();
+            tot += t2;
         }
-        // the part's rows in this batch, and this wave's share [pos, stop) of them
-        const uint32_t blo = plo > base ? (uint32_t)(plo - base < tot ? plo - base : tot) : 0u;
-        const uint32_t bhi = phi - base < tot ? (uint32_t)(phi - base) : tot;
-        const uint32_t nb = bhi > blo ? bhi - blo : 0u;
-        base += tot;
-        uint64_t share = ((uint64_t)nb + NT / 64 - 1) / (NT / 64);
-        share = (share + kBStep - 1) / kBStep * kBStep;
-        const uint64_t wlo = wave * share < nb ? wave * share : nb;
-        const uint64_t whi = wlo + share < nb ? wlo + share : nb;
-        uint32_t pos = uni(blo + (uint32_t)wlo);
-        const uint32_t stop = uni(blo + (uint32_t)whi);
-        // the lattice row that holds row `pos` of the batch: rows [.., kend) of the batch
-        // are in it or before it, and row j in it is row j + kdelta of the sorted set
-        int32_t k = 0;
-        if (pos < stop) {
-            int32_t top = 1;
-            while (2 * top < nr) top *= 2;
+        b_region_init(smem, L, threadIdx.x, NT);
+        __syncthreads();
+        // this part's rows [lo, hi) of the tile's rows
+        const unsigned long long E = d.nparts > 1 ? (tot + d.nparts - 1) / d.nparts : tot;
+        unsigned long long lo = (unsigned long long)m.part * E, hi = lo + E;
+        lo = lo < tot ? lo : tot;
+        hi = hi < tot ? hi : tot;
+        const int32_t nr = nrow;
+        int32_t top = 1;  // binary search over the table: the largest power of two < nr
+        while (2 * top < nr) top *= 2;
+        // the last lattice row starting at or before j
+        auto row_of = [&](unsigned long long j) {
+            int32_t k = 0;
             for (int32_t step = top; step >= 1; step >>= 1)
-                if (k + step < nr && uni(s_pre[k + step]) <= pos) k += step;
-        }
-        uint32_t kend = 0, kdelta = 0;
-        auto enter = [&]() {
-            kend = k + 1 < nr ? uni(s_pre[k + 1]) : tot;
-            kdelta = uni(s_start[k] - s_pre[k]);
+                if (k + step < nr && (unsigned long long)s_pre[k + step] <= j) k += step;
+            return k;
         };
-        if (pos < stop) enter();
-        using R = BRows<VAL>;
-        auto load = [&](R &S) {
-            S.row = S.end = 0;
-            if (pos < stop) {  // uniform
-                while (pos >= kend) { ++k; enter(); }  // (lattice rows may be empty)
-                uint32_t n = (kend < stop ? kend : stop) - pos;
-                n = n < (uint32_t)kBStep ? n : (uint32_t)kBStep;
-                S.row = pos + kdelta;
-                S.end = S.row + n;
-                pos += n;
+        // Each thread keeps a run of rows that land in one cell in registers and adds it to
+        // the LDS region when the cell changes: the rows are sorted by lattice cell, so in
+        // a dense view a thread's rows (NT apart) fall in one pixel for long stretches, and
+        // the run replaces per-row LDS atomics that would all hit the same address.
+        uint32_t run_lc = 0, run_n = 0, run_nan = 0;
+        double run_s = 0.0;
+        auto flush = [&]() {
+            if (run_n == 0u) return;
+            atomicAdd(reinterpret_cast<uint32_t *>(smem + L.o_cnt) + run_lc, run_n);
+            if (L.has_val) {
+                if (run_nan) atomicAdd(reinterpret_cast<uint32_t *>(smem + L.o_nan) + run_lc, run_nan);
+                if (run_n > run_nan) atomicAdd(reinterpret_cast<double *>(smem + L.o_sum) + run_lc, run_s);
             }
-            S.load(A, lane);
+            run_n = 0u;
+            run_nan = 0u;
+            run_s = 0.0;
         };
-        auto bin = [&](const R &S) {
-            if (S.row == S.end) return;  // uniform
-            const uint32_t r0 = S.row + 4u * (uint32_t)lane, a0 = S.at(A, lane);
-            uint32_t lc[4];
-            bool keep[4];
+        // project kBItems loaded rows and add the tile's ones to the thread's run
+        auto bin = [&](const float *xs, const float *ys, const float *vs, const bool *ok) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const double x = (double)S.x[e], y = (double)S.y[e];
-                const uint32_t r = a0 + (uint32_t)e;
-                const bool in = (q.xmin <= x) & (x <= q.xmax) & (q.ymin <= y) & (y <= q.ymax);
-                // (the conversion saturates; a row out of the view is dropped by `in`)
-                int32_t xx, yy;
-                asm("v_cvt_i32_f64 %0, %1" : "=v"(xx) : "v"(__dadd_rn(__dmul_rn(x, q.sx), q.tx)));
-                asm("v_cvt_i32_f64 %0, %1" : "=v"(yy) : "v"(__dadd_rn(__dmul_rn(y, q.sy), q.ty)));
+            for (int it = 0; it < kBItems; ++it) {
+                if (!ok[it]) continue;
+                const double x = (double)xs[it], y = (double)ys[it];
+                if (!((q.xmin <= x && x <= q.xmax) && (q.ymin <= y && y <= q.ymax))) continue;
+                int32_t xx = proj(x, q.sx, q.tx), yy = proj(y, q.sy, q.ty);
                 xx = xx >= q.W ? q.W - 1 : xx;
                 yy = yy >= q.H ? q.H - 1 : yy;
-                xx += xx < 0 ? q.W : 0;  // numba's negative-index wraparound
-                yy += yy < 0 ? q.H : 0;
-                const uint32_t cx = (uint32_t)(xx - px0), cy = (uint32_t)(yy - py0);
-                keep[e] = (r >= r0) & (r < S.end) & in & (cx < tw) & (cy < th);
-                lc[e] = ((cy * (uint32_t)q.tw + cx) << cl) | mine;  // this lane's copy
-            }
-            if (!__any(keep[0] | keep[1] | keep[2] | keep[3])) return;
-            const bool same4 = keep[0] & keep[1] & keep[2] & keep[3] & (lc[0] == lc[1]) &
-                               (lc[0] == lc[2]) & (lc[0] == lc[3]);
-            if (__all(same4)) {
-                uint32_t nan = 0;
-                double s = 0.0;
-                if constexpr (VAL) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const double v = (double)S.v[e];
-                        if (v != v) ++nan;
-                        else s += v;
-                    }
+                if (xx < 0) xx += q.W;  // numba's negative-index wraparound
+                if (yy < 0) yy += q.H;
+                if (xx < px0 || xx >= px1 || yy < py0 || yy >= py1) continue;  // another tile's
+                const uint32_t lc = (uint32_t)((yy - py0) * q.tw + (xx - px0));
+                if (lc != run_lc) {
+                    flush();
+                    run_lc = lc;
                 }
-                if (__all(lc[0] >> cl == uni(lc[0] >> cl))) {  // the whole step in one pixel
-                    if constexpr (VAL) {
-                        for (int off = 32; off > 0; off >>= 1) {
-                            s += __shfl_xor(s, off, 64);
-                            nan += __shfl_xor(nan, off, 64);
-                        }
-                    }
-                    if (lane == 0) {
-                        atomicAdd(l_cnt + lc[0], (uint32_t)kBStep);
-                        if constexpr (VAL) {
-                            if (nan) atomicAdd(l_nan + lc[0], nan);
-                            atomicAdd(l_sum + lc[0], s);
-                        }
-                    }
-                    return;
-                }
-                atomicAdd(l_cnt + lc[0], 4u);
-                if constexpr (VAL) {
-                    if (nan) atomicAdd(l_nan + lc[0], nan);
-                    atomicAdd(l_sum + lc[0], s);
-                }
-                return;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (!keep[e]) continue;
-                atomicAdd(l_cnt + lc[e], 1u);
-                if constexpr (VAL) {
-                    const double v = (double)S.v[e];
-                    if (v != v) atomicAdd(l_nan + lc[e], 1u);
-                    else atomicAdd(l_sum + lc[e], v);
+                ++run_n;
+                if (L.has_val) {
+                    const double v = (double)vs[it];
+                    if (v != v) ++run_nan;
+                    else run_s += v;
                 }
             }
         };
-        if (pos < stop) {  // uniform in the wave; no barrier inside
-            R ra, rb, rc;  // three register sets rotate roles
-            load(ra);
-            load(rb);
-            do {  // no exit between the steps: one past the share loads row 0 and bins nothing
-                load(rc);
-                bin(ra);
-                load(ra);
-                bin(rb);
-                load(rb);
-                bin(rc);
-            } while (ra.row != ra.end);
+        // Rows [lo, hi) of the tile's concatenated lattice rows, NT * kBItems a chunk, the
+        // next chunk's loads issued before this chunk is binned.  A chunk that lies inside
+        // one lattice row (the common case for a wide view, whose lattice rows are long)
+        // is one contiguous run of sorted rows, found by one search for the whole chunk;
+        // any other chunk finds each row's lattice row by a search of the table.
+        struct Set {
+            float x[kBItems], y[kBItems], v[kBItems];
+            bool ok[kBItems];
+        };
+        auto load = [&](unsigned long long c, Set &S) {
+            const int32_t kc = row_of(c < tot ? c : (tot > 0 ? tot - 1 : 0));  // uniform
+            const unsigned long long kend = kc + 1 < nr ? (unsigned long long)s_pre[kc + 1] : tot;
+            const bool one = c + (unsigned long long)(NT * kBItems) <= kend;   // uniform
+#pragma unroll
+            for (int it = 0; it < kBItems; ++it) {
+                const unsigned long long j = c + (unsigned long long)(it * NT + threadIdx.x);
+                S.ok[it] = j < hi;
+                int64_t row;
+                if (one) {  // j < kend: a row of lattice row kc (read even past hi, dropped)
+                    row = (int64_t)s_start[kc] + (int64_t)(j - s_pre[kc]);
+                } else {
+                    const unsigned long long jj = S.ok[it] ? j : lo;  // past hi: row lo, dropped
+                    const int32_t k = row_of(jj);
+                    row = (int64_t)s_start[k] + (int64_t)(jj - s_pre[k]);
+                }
+                S.x[it] = A.x[row];
+                S.y[it] = A.y[row];
+                S.v[it] = L.has_val ? A.v[row] : 0.0f;
+            }
+        };
+        if (lo < hi) {
+            constexpr unsigned long long kStep = (unsigned long long)NT * kBItems;
+            Set sa, sb;
+            load(lo, sa);
+            // no exit between the two halves: a step past hi loads row lo and bins nothing
+            for (unsigned long long c = lo; c < hi; c += 2 * kStep) {
+                load(c + kStep, sb);
+                bin(sa.x, sa.y, sa.v, sa.ok);
+                load(c + 2 * kStep, sa);
+                bin(sb.x, sb.y, sb.v, sb.ok);
+            }
         }
-        }
+        flush();
         __syncthreads();
         if (d.nparts > 1) {
-            // a split tile's part: the tile's cells go to scratch (one copy each), the merge
-            // kernel folds the parts
+            // a split tile's part: the tile's cells of its region go to scratch (same
+            // layout), the merge kernel folds them
             if (d.region + m.part < (uint32_t)A.max_regions) {
                 uint8_t *dst = A.scratch + (size_t)(d.region + m.part) * L.bytes;
                 const uint32_t used = (uint32_t)(q.tw * q.th);
                 for (uint32_t c = threadIdx.x; c < used; c += NT) {
-                    uint32_t n, nn;
-                    double sum;
-                    b_fold_cell(smem, L, c, cl, n, nn, sum);
-                    reinterpret_cast<uint32_t *>(dst + L.o_cnt)[c] = n;
-                    if constexpr (VAL) {
-                        reinterpret_cast<uint32_t *>(dst + L.o_nan)[c] = nn;
-                        reinterpret_cast<double *>(dst + L.o_sum)[c] = sum;
+                    reinterpret_cast<uint32_t *>(dst + L.o_cnt)[c] = reinterpret_cast<const uint32_t *>(smem + L.o_cnt)[c];
+                    if (L.has_val) {
+                        reinterpret_cast<uint32_t *>(dst + L.o_nan)[c] = reinterpret_cast<const uint32_t *>(smem + L.o_nan)[c];
+                        reinterpret_cast<double *>(dst + L.o_sum)[c] = reinterpret_cast<const double *>(smem + L.o_sum)[c];
                     }
                 }
             }
         } else {
-            b_store_tile(smem, L, cl, q, d.t, NT);
+            b_store_tile(smem, L, q, d.t, NT);
         }
-        // (the region and table are rebuilt for the next item after the loop's barrier)
-        if (threadIdx.x == 0) s_item = next;
+        __syncthreads();  // the region and table are rebuilt for the next item
     }
 }
 
 // ---- merge: split tiles ---------------------------------------------------------------
-// kBMergeThreads cells of a split tile per workgroup, one a thread: a heavy tile has many
-// parts, so its cells are spread over the chip (one workgroup per tile left 8 of 256 CUs
-// with all the parts of a 256 x 256 canvas; 24 viewports over 100M rows: 339 -> 65 us).
-constexpr int kBMergeThreads = 256;
+constexpr int kBMergeThreads = 512;
 
 __global__ __launch_bounds__(kBMergeThreads) void b_merge_kernel(BArgs A) {
+    extern __shared__ __align__(16) uint8_t smem[];
     const BLay &L = A.L;
-    const uint32_t nsplit = A.ctr[2] < (uint32_t)A.max_tiles ? A.ctr[2] : (uint32_t)A.max_tiles;
-    const uint32_t nch = (L.cap + kBMergeThreads - 1) / kBMergeThreads;
-    for (uint32_t i = blockIdx.x; i < nsplit * nch; i += gridDim.x) {
-        const BTile d = A.tiles[A.split[i / nch]];
+    const uint32_t nsplit = A.ctr[2];
+    for (uint32_t s = blockIdx.x; s < nsplit && s < (uint32_t)A.max_tiles; s += gridDim.x) {
+        const BTile d = A.tiles[A.split[s]];
         const BReq q = A.reqs[d.req];
-        const uint32_t c = (i % nch) * kBMergeThreads + threadIdx.x;
-        int32_t px0, px1, py0, py1;
-        b_tile_rect(q, d.t, px0, px1, py0, py1);
-        const int32_t ly = (int32_t)(c / (uint32_t)q.tw), lx = (int32_t)(c - (uint32_t)ly * (uint32_t)q.tw);
-        if (ly >= py1 - py0 || lx >= px1 - px0) continue;  // not a cell of the tile
         const uint32_t np = d.region + d.nparts <= (uint32_t)A.max_regions ? d.nparts : 0u;
         const uint8_t *parts = A.scratch + (size_t)d.region * L.bytes;
-        constexpr uint32_t kU = 8;                     // parts whose loads are in flight together
-        uint32_t n = 0, nn = 0;
-        double sum = 0.0;
-        uint32_t p = 0;
-        for (; p + kU <= np; p += kU) {
-            uint32_t cn[kU], cnn[kU];
-            double cs[kU];
+        const uint32_t used = (uint32_t)(q.tw * q.th);  // the tile's cells of each region
+        constexpr uint32_t kU = 4;                     // parts whose loads are in flight together
+        for (uint32_t c = threadIdx.x; c < used; c += kBMergeThreads) {
+            uint32_t n = 0, nn = 0;
+            double sum = 0.0;
+            uint32_t p = 0;
+            for (; p + kU <= np; p += kU) {
+                uint32_t cn[kU], cnn[kU];
+                double cs[kU];
 #pragma unroll
-            for (uint32_t u = 0; u < kU; ++u) {
-                const uint8_t *r = parts + (size_t)(p + u) * L.bytes;
-                cn[u] = reinterpret_cast<const uint32_t *>(r + L.o_cnt)[c];
-                cnn[u] = L.has_val ? reinterpret_cast<const uint32_t *>(r + L.o_nan)[c] : 0u;
-                cs[u] = L.has_val ? reinterpret_cast<const double *>(r + L.o_sum)[c] : 0.0;
-            }
+                for (uint32_t u = 0; u < kU; ++u) {
+                    const uint8_t *r = parts + (size_t)(p + u) * L.bytes;
+                    cn[u] = reinterpret_cast<const uint32_t *>(r + L.o_cnt)[c];
+                    cnn[u] = L.has_val ? reinterpret_cast<const uint32_t *>(r + L.o_nan)[c] : 0u;
+                    cs[u] = L.has_val ? reinterpret_cast<const double *>(r + L.o_sum)[c] : 0.0;
+                }
 #pragma unroll
-            for (uint32_t u = 0; u < kU; ++u) {
-                n += cn[u];
-                nn += cnn[u];
-                sum += cs[u];
+                for (uint32_t u = 0; u < kU; ++u) {
+                    n += cn[u];
+                    nn += cnn[u];
+                    sum += cs[u];
+                }
             }
-        }
-        for (; p < np; ++p) {
-            const uint8_t *r = parts + (size_t)p * L.bytes;
-            n += reinterpret_cast<const uint32_t *>(r + L.o_cnt)[c];
+            for (; p < np; ++p) {
+                const uint8_t *r = parts + (size_t)p * L.bytes;
+                n += reinterpret_cast<const uint32_t *>(r + L.o_cnt)[c];
+                if (L.has_val) {
+                    nn += reinterpret_cast<const uint32_t *>(r + L.o_nan)[c];
+                    sum += reinterpret_cast<const double *>(r + L.o_sum)[c];
+                }
+            }
+            reinterpret_cast<uint32_t *>(smem + L.o_cnt)[c] = n;
             if (L.has_val) {
-                nn += reinterpret_cast<const uint32_t *>(r + L.o_nan)[c];
-                sum += reinterpret_cast<const double *>(r + L.o_sum)[c];
+                reinterpret_cast<uint32_t *>(smem + L.o_nan)[c] = nn;
+                reinterpret_cast<double *>(smem + L.o_sum)[c] = sum;
             }
         }
-        b_store_values(q, (int64_t)(py0 + ly) * q.W + (px0 + lx), L.has_val, n, nn, sum);
+        __syncthreads();
+        b_store_tile(smem, L, q, d.t, kBMergeThreads);
+        __syncthreads();
     }
 }
 
@@ -721,7 +598,7 @@ struct BLayout {
 static int b_plan(const dsx_batch_config *c, BLayout &P) {
     if (!c) return DSX_ERR_NULL;
     if (c->max_requests < 1 || c->max_tiles < 1 || c->max_regions < 1) return DSX_ERR_SHAPE;
-    if (c->grid < 1 || c->grid > kBMaxGrid || c->n < 0) return DSX_ERR_SHAPE;
+    if (c->grid < 1 || c->grid > kBMaxLatRows || c->n < 0) return DSX_ERR_SHAPE;
     if (c->n >= (1ll << 32)) return DSX_ERR_SHAPE;  // the tile tables hold 32-bit rows
     if (!(c->x1 > c->x0) || !(c->y1 > c->y0)) return DSX_ERR_SHAPE;
     if (c->planes == 0 || (c->planes & ~(uint32_t)(BP_COUNT | BP_COUNTV | BP_SUM | BP_MEAN)))
@@ -732,9 +609,7 @@ static int b_plan(const dsx_batch_config *c, BLayout &P) {
     if (c->threads != 256 && c->threads != 512 && c->threads != 1024) return DSX_ERR_SHAPE;
     if (c->workgroups < 1) return DSX_ERR_SHAPE;
     const uint32_t cb = has_val ? 16u : 4u;
-    // a workgroup's share of the CU's LDS by its threads: 1024 / threads workgroups fit a CU,
-    // so that one streams rows while another starts or stores its tile
-    const uint32_t cap = (uint32_t)((kBLds * (c->threads / 256) / 4 - kBTable - 512) / cb) & ~3u;
+    const uint32_t cap = (uint32_t)((kBLds - kBTable - 1024) / cb) & ~3u;
     P.L = b_layout(has_val, cap);
     P.max_regions = c->max_regions;
     P.max_items = c->max_tiles + c->max_regions;
@@ -769,12 +644,6 @@ struct dsx_batch {
     int use_graph;
 };
 
-static decltype(&b_agg_kernel<1024, true>) b_agg_of(int32_t threads, bool has_val) {
-    if (threads == 256) return has_val ? b_agg_kernel<256, true> : b_agg_kernel<256, false>;
-    if (threads == 512) return has_val ? b_agg_kernel<512, true> : b_agg_kernel<512, false>;
-    return has_val ? b_agg_kernel<1024, true> : b_agg_kernel<1024, false>;
-}
-
 static int b_launch_all(dsx_batch *b, hipStream_t st) {
     const BArgs &A = b->A;
     const dsx_batch_config &c = b->cfg;
@@ -789,8 +658,13 @@ static int b_launch_all(dsx_batch *b, hipStream_t st) {
     hipLaunchKernelGGL(b_tiles_kernel, dim3(tg), dim3(kBTileThreads), 0, st, A);
     hipLaunchKernelGGL(b_items_kernel, dim3(1), dim3(kBItemThreads), 0, st, A);
     const size_t lds = (size_t)b->P.L.bytes + kBTable;
-    hipLaunchKernelGGL(b_agg_of(c.threads, b->P.L.has_val), dim3(c.workgroups), dim3(c.threads), lds, st, A);
-    hipLaunchKernelGGL(b_merge_kernel, dim3(2048), dim3(kBMergeThreads), 0, st, A);
+    switch (c.threads) {
+    case 256: hipLaunchKernelGGL(b_agg_kernel<256>, dim3(c.workgroups), dim3(256), lds, st, A); break;
+    case 512: hipLaunchKernelGGL(b_agg_kernel<512>, dim3(c.workgroups), dim3(512), lds, st, A); break;
+    default: hipLaunchKernelGGL(b_agg_kernel<1024>, dim3(c.workgroups), dim3(1024), lds, st, A); break;
+    }
+    const int mg = c.max_tiles < 1024 ? c.max_tiles : 1024;
+    hipLaunchKernelGGL(b_merge_kernel, dim3(mg), dim3(kBMergeThreads), (size_t)b->P.L.bytes, st, A);
     return launch_status();
 }
 
@@ -856,8 +730,14 @@ extern "C" int dsx_batch_create(const dsx_batch_config *c, void *workspace, size
     A.cs = c->cell_start;
     A.planes = c->planes;
     const int lds = (int)(P.L.bytes + kBTable);
-    e = hipFuncSetAttribute((const void *)b_agg_of(c->threads, P.L.has_val),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const void *kerns[3] = {(const void *)b_agg_kernel<256>, (const void *)b_agg_kernel<512>,
+                            (const void *)b_agg_kernel<1024>};
+    for (const void *k : kerns) {
+        e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) { record_hip_error(e); delete b; return DSX_ERR_HIP; }
+    }
+    e = hipFuncSetAttribute((const void *)b_merge_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)P.L.bytes);
     if (e != hipSuccess) { record_hip_error(e); delete b; return DSX_ERR_HIP; }
     b->use_graph = use_graph ? 1 : 0;
     b->graph = nullptr;
