@@ -2,7 +2,7 @@
 // as a tiled LDS engine for gfx950.
 //
 // Device-scope global atomics run at ~27 G/s on this part while LDS atomics run at
-// ~780 G/s (u32 and f64 alike), so no per-row update touches a global atomic:
+// 5.1 T/s (u32) and 1.8 T/s (f64) over the chip, so no per-row update touches a global atomic:
 //
 //   select   a sampled coarse density histogram picks the hot rectangle ("window")
 //            of the canvas whose aggregate planes fit the 160 KB LDS of a workgroup
