@@ -123,10 +123,17 @@ __device__ __forceinline__ bool unclipped(double v0, double d, double lo, double
     return __dsub_rn(v0, lo) >= -d && __dsub_rn(hi, v0) >= d;
 }
 
-// draw_segment, line.py:1045-1095, for coordinates of column types TX / TY.
-template <typename TX, typename TY, typename I, typename S>
-__device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bool segment_start,
-                                             TX x0c, TX x1c, TY y0c, TY y1c) {
+// The pixels a segment is drawn between, what is left of it in the view.
+struct Ends {
+    int32_t x0, y0, x1, y1;
+    bool start, clipped;
+};
+
+// draw_segment, line.py:1045-1095, up to its _bresenham call, for coordinates of column
+// types TX / TY: false where nothing is drawn.
+template <typename TX, typename TY>
+__device__ __forceinline__ bool segment_ends(const LineArgs &a, bool segment_start, TX x0c, TX x1c,
+                                             TY y0c, TY y1c, Ends &e) {
     double x0 = (double)x0c, x1 = (double)x1c, y0 = (double)y0c, y1 = (double)y1c;
     bool skip = (x0 != x0) || (y0 != y0) || (x1 != x1) || (y1 != y1);
     if (x0 < a.xmin && x1 < a.xmin) skip = true;
@@ -147,16 +154,17 @@ __device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bo
         if (!clipt(-dy1, __dsub_rn(y0, a.ymin), t0, t1)) skip = true;
         if (!clipt(dy1, __dsub_rn(a.ymax, y0), t0, t1)) skip = true;
     }
-    if (skip) return;
-    bool clipped = false;
+    if (skip) return false;
+    e.start = segment_start;
+    e.clipped = false;
     if (t1 < 1) {
-        clipped = true;
+        e.clipped = true;
         x1 = __dadd_rn(x0, __dmul_rn(t1, dx1));
         y1 = __dadd_rn(y0, __dmul_rn(t1, dy1));
     }
     if (t0 > 0) {
-        clipped = true;
-        segment_start = true;
+        e.clipped = true;
+        e.start = true;
         x0 = __dadd_rn(x0, __dmul_rn(t0, dx1));
         y0 = __dadd_rn(y0, __dmul_rn(t0, dy1));
     }
@@ -164,13 +172,20 @@ __device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bo
     const int64_t py0 = snap1(y0, a.sy, a.ty, a.yymax, a.ylog);
     const int64_t px1 = snap1(x1, a.sx, a.tx, a.xxmax, a.xlog);
     const int64_t py1 = snap1(y1, a.sy, a.ty, a.yymax, a.ylog);
+    e.x0 = (int32_t)px0; e.y0 = (int32_t)py0; e.x1 = (int32_t)px1; e.y1 = (int32_t)py1;
     // Clipped ends project into [0, W] x [0, H] (one pixel of rounding slack either
     // side); anything else comes from a degenerate view (infinite or NaN scale) and
     // would make the walk unbounded, so such a segment is not drawn.
-    if (px0 < -1 || px0 > a.W + 1 || px1 < -1 || px1 > a.W + 1 || py0 < -1 ||
-        py0 > a.H + 1 || py1 < -1 || py1 > a.H + 1)
-        return;
-    put.template walk<I>(segment_start, (I)px0, (I)px1, (I)py0, (I)py1, clipped);
+    return !(px0 < -1 || px0 > a.W + 1 || px1 < -1 || px1 > a.W + 1 || py0 < -1 ||
+             py0 > a.H + 1 || py1 < -1 || py1 > a.H + 1);
+}
+
+template <typename TX, typename TY, typename I, typename S>
+__device__ __forceinline__ void draw_segment(const LineArgs &a, const S &put, bool segment_start,
+                                             TX x0c, TX x1c, TY y0c, TY y1c) {
+    Ends e;
+    if (segment_ends<TX, TY>(a, segment_start, x0c, x1c, y0c, y1c, e))
+        put.template walk<I>(e.start, (I)e.x0, (I)e.x1, (I)e.y0, (I)e.y1, e.clipped);
 }
 
 template <typename TX, typename TY, typename TV, bool HAS_VAL, bool SQDEV>
@@ -237,30 +252,34 @@ struct Box {
     }
 };
 
-// _bresenham for an unclipped segment whose ends (so all its pixels) lie in the box.  With
-// n steps along the major axis and m <= n along the minor one, the reference's error term
-// has moved the minor axis floor((2 m i + n - b) / 2 n) times after i steps, b = 1 where
-// the major axis runs backwards (its tie rule), else 0.  Short segments hold that quotient,
-// moved up by 1 / 4n -- half of its distance to the next value above --, in fixed point with
-// 20 fractional bits: n steps of a slope that is off by less than 1.5 * 2^-20 stay within
-// 1 / 4n for n < kDdaMax, so the floor is exact.  A step is then an add, a shift, a
-// multiply-add and an add, with no compare or select.  Long ones keep the error term (its
-// half, less b, so that the reference's `err >= 0 && (err || i > 0)` is err >= 0).
+// _bresenham for a segment whose ends (so all its pixels) lie in the box; first: whether
+// its first pixel is drawn.  With n steps along the major axis and m <= n along the minor
+// one, the reference's error term has moved the minor axis floor((2 m i + n - b) / 2 n)
+// times after i steps, b = 1 where the major axis runs backwards (its tie rule), else 0.
+// Short segments hold that quotient, moved up by 1 / 4n -- half of its distance to the next
+// value above --, in fixed point with 20 fractional bits: n steps of a slope that is off by
+// less than 1.5 * 2^-20 stay within 1 / 4n for n < kDdaMax, so the floor is exact.  A step
+// is then an add, a shift, a multiply-add and an add, with no compare or select.  Long ones
+// keep the error term (its half, less b, so that the reference's
+// `err >= 0 && (err || i > 0)` is err >= 0), and so do the short ones of a wave that has a
+// long one: their loops would run one after the other (100k x 256 samples of white noise,
+// where nearly every wave has both and a clipped one, into 2048 x 1024: 19.9 ms with a loop
+// for each kind, 5.0 with one).
 // common: a number of steps that every active lane takes (uniform), so that those run
 // without a lane mask.
 constexpr int32_t kDdaMax = 256;
 
 __device__ __forceinline__ void box_walk(uint32_t at, int32_t dx, int32_t dy, uint32_t pitch4,
-                                         bool start, int32_t common) {
+                                         bool first, int32_t common) {
     const int32_t ax = dx < 0 ? -dx : dx, ay = dy < 0 ? -dy : dy;
     const bool xm = ax >= ay;
     const int32_t n = xm ? ax : ay, m = xm ? ay : ax;
-    if (start || n == 0) box_add(at);
+    if (first) box_add(at);
     const int32_t ox = dx < 0 ? -4 : 4, oy = dy < 0 ? -(int32_t)pitch4 : (int32_t)pitch4;
     const int32_t o1 = xm ? ox : oy, o2 = xm ? oy : ox;  // along the major axis; the minor
     const bool fwd = (xm ? dx : dy) > 0;
-    if (n < kDdaMax) {
-        const float rn = __builtin_amdgcn_rcpf((float)n);
+    if (!__any(n >= kDdaMax)) {
+        const float rn = __builtin_amdgcn_rcpf((float)n);  // (n = 0: nothing is read of it)
         const uint32_t slope = (uint32_t)((float)m * rn * 1048576.0f);
         const int32_t quarter = (int32_t)(rn * 262144.0f);
         uint32_t acc = 524288u + (uint32_t)(fwd ? quarter : -quarter);
@@ -339,7 +358,7 @@ __device__ __forceinline__ void box_flush(const Box &b, uint32_t *count, int32_t
 // projected once (not once per segment it ends), in 32 bits, and only segments that
 // clipping could shorten take draw_segment: telling those by an inexact float32 delta sent
 // a lane of nearly every wave there (values near zero), 2.21 against 1.54 ms.  The
-// fixed-point walk, its common steps without a lane mask: 1.54 -> 1.10 ms.  Before all of
+// fixed-point walk, its common steps without a lane mask: 1.54 -> 1.12 ms.  Before all of
 // it 2.89 ms (2048 x 1024).
 constexpr int kStripMaxK = 8;        // segments per strip
 
@@ -436,7 +455,8 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
         bool gap = j0 == 0 || row.prev != row.prev;  // the sample before is missing
         double y0 = (double)row.y[0];
         bool in0 = a.ymin <= y0 && y0 <= a.ymax;
-        int32_t py0 = snap_in<LOG>(y0, a.sy, a.ty, yymax, a.ylog);
+        // (a log10 of nothing in the view is not worked out)
+        int32_t py0 = !LOG || in0 ? snap_in<LOG>(y0, a.sy, a.ty, yymax, a.ylog) : -1;
         int4 g = *reinterpret_cast<const int4 *>(&s_seg[0]);  // px0, px1, flags
         // segments drawn from the front of a shifting register window (a rolled loop with
         // constant register indices: one copy of the rasteriser, no indexed registers)
@@ -449,22 +469,37 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
             const TY y0c = row.y[0], y1c = row.y[1];
             const double y1 = (double)y1c;
             const bool in1 = a.ymin <= y1 && y1 <= a.ymax;
-            const int32_t py1 = snap_in<LOG>(y1, a.sy, a.ty, yymax, a.ylog);
+            const int32_t py1 = !LOG || in1 ? snap_in<LOG>(y1, a.sy, a.ty, yymax, a.ylog) : -1;
             const bool start = gap || (flags & SEG_START) != 0;
             const bool fast = in0 & in1 & ((uint32_t)py0 < (uint32_t)a.H) &
                               ((uint32_t)py1 < (uint32_t)a.H) &
                               unclipped(y0, (double)(TY)(y1c - y0c), a.ymin, a.ymax) &
                               ((flags & SEG_FAST) != 0);
-            const int32_t dx = px1 - px0;
-            if (fast) {
-                box_walk(put.box.at(px0, py0), dx, py1 - py0, pitch4, start, dx < 0 ? -dx : dx);
-            } else if (!(flags & SEG_SKIP)) {
-                // (both ends beyond one bound, or one missing: nothing is drawn)
-                const bool none = y0 != y0 || y1 != y1 || (y0 < a.ymin && y1 < a.ymin) ||
-                                  (y0 > a.ymax && y1 > a.ymax);
-                if (!none)
-                    draw_segment<TX, TY, int32_t>(a, put, start, (TX)s_seg[q].x0, (TX)s_seg[q].x1,
-                                                  y0c, y1c);
+            const bool first = start || (px0 == px1 && py0 == py1);
+            // (a copy of its own, so that the x side of the walk stays in scalar registers: 1M x
+            // 256 series 1.20 ms with the ends in the vector registers of the other, 1.12 so)
+            if (__all(fast)) {
+                const int32_t dx = px1 - px0;
+                box_walk(put.box.at(px0, py0), dx, py1 - py0, pitch4, first, dx < 0 ? -dx : dx);
+            } else {
+                // each lane's own pixels or what clipping leaves of them, then one walk for
+                // the lanes of either kind
+                Ends e{px0, py0, px1, py1, first, false};
+                bool draw = fast;
+                if (!fast && !(flags & SEG_SKIP)) {
+                    // (both ends beyond one bound, or one missing: nothing is drawn)
+                    const bool none = y0 != y0 || y1 != y1 || (y0 < a.ymin && y1 < a.ymin) ||
+                                      (y0 > a.ymax && y1 > a.ymax);
+                    if (!none && segment_ends<TX, TY>(a, start, (TX)s_seg[q].x0, (TX)s_seg[q].x1,
+                                                      y0c, y1c, e)) {
+                        draw = put.box.has(e.x0, e.y0) && put.box.has(e.x1, e.y1) && e.x0 < a.W &&
+                               e.x1 < a.W;
+                        if (!draw) put.walk<int32_t>(e.start, e.x0, e.x1, e.y0, e.y1, e.clipped);
+                        e.start = e.start || (!e.clipped && e.x0 == e.x1 && e.y0 == e.y1);
+                    }
+                }
+                if (draw)
+                    box_walk(put.box.at(e.x0, e.y0), e.x1 - e.x0, e.y1 - e.y0, pitch4, e.start, 0);
             }
             gap = y0 != y0;
             y0 = y1;
@@ -616,7 +651,7 @@ __global__ __launch_bounds__(kBoxThreads) void lines_run_kernel(LineArgs a, uint
                                    : (xpc[u] != xpc[u]) || (ypc[u] != ypc[u]);
             if ((whole >> u & 1u) && put.box.has(px0[u], py0[u]) && put.box.has(px1[u], py1[u]))
                 box_walk(put.box.at(px0[u], py0[u]), px1[u] - px0[u], py1[u] - py0[u], pitch4,
-                         start, 0);
+                         start || (px0[u] == px1[u] && py0[u] == py1[u]), 0);
             else
                 draw_segment<TX, TY, int32_t>(a, put, start, x0c[u], x1c[u], y0c[u], y1c[u]);
         }
