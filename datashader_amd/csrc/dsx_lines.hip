@@ -689,11 +689,22 @@ static int launch_strips(const LineArgs &a, uint32_t *count, int64_t nstrips, in
 template <typename TX, typename TY>
 static int launch_runs(const LineArgs &a, uint32_t *count, hipStream_t s) {
     const int64_t nseg = a.nverts - 1;
-    // about one workgroup per CU (its box takes the CU's LDS), of at least 256 segments (20k
-    // segments: 1024 each 61.9 us a call, 256 each 59.8)
-    int64_t groups = (cu_count() + a.nlines - 1) / a.nlines;
+    // at most one workgroup per CU (its box takes the CU's LDS), of at least 256 segments (20k
+    // segments: 1024 each 61.9 us a call, 256 each 59.8).  Where the lines alone are more
+    // than that, a last round of few workgroups leaves the chip idle: lines are then split
+    // as long as that shortens the rounds' sum and a workgroup keeps half a round of segments
+    // (300 lines of 12000 noisy vertices, 300 workgroups on 256 CUs: 15.9 ms, 6.3
+    // split; one global atomic a pixel 13.6).
+    const int64_t cus = cu_count();
+    int64_t groups = cus / a.nlines;
     const int64_t most = (nseg + 255) / 256;
     groups = groups > most ? most : groups;
+    if (groups < 1) {
+        groups = 1;
+        const auto rounds = [&](int64_t g) { return (a.nlines * g + cus - 1) / cus; };
+        for (int64_t g = 2; g <= 8 && nseg >= g * (kRunSegs / 2); ++g)
+            if (rounds(g) * groups < rounds(groups) * g) groups = g;
+    }
     const int64_t per = (nseg + groups - 1) / groups;
     auto kern = a.xlog || a.ylog ? lines_run_kernel<TX, TY, true> : lines_run_kernel<TX, TY, false>;
     constexpr int lds = kBoxLds + 64;  // the box and a round's bounds
