@@ -182,17 +182,17 @@ class DeviceFrame:
                 continue  # non-numeric columns stay on the host (never aggregated)
         floats = {name: df[name].to_numpy() for names in groups.values() for name in names}
         nbytes = sum(a.nbytes for a in (*plain.values(), *floats.values()))
-        if torch.device(device).type == "cuda" and nbytes >= _upload.MIN_BYTES:
-            pairs = []
+        if torch.device(device).type == "cuda" and _upload.worth(nbytes, len(plain) + len(floats)):
+            blocks = []
             for name, a in plain.items():
                 cols[name] = torch.empty(len(df), dtype=_torch_dtype(a.dtype), device=device)
-                pairs.append((a, cols[name]))
+                blocks.append(([a], cols[name]))
             for dt, names in groups.items():
                 block = torch.empty((len(names), len(df)), dtype=_torch_dtype(dt), device=device)
                 for j, name in enumerate(names):
                     cols[name] = block[j]
-                    pairs.append((floats[name], block[j]))
-            _upload.upload(pairs)
+                blocks.append(([floats[name] for name in names], block))
+            _upload.upload(blocks)
         else:
             for name, a in plain.items():
                 cols[name] = torch.from_numpy(np.ascontiguousarray(a)).to(device)
