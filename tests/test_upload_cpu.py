@@ -12,8 +12,9 @@ def _blocks(shapes, rng):
     out = []
     for dt, ncols, n in shapes:
         a = rng.integers(0, 100, (ncols, n)).astype(dt)
-        out.append(([np.asfortranarray(a)[j] if ncols > 1 else a[j] for j in range(ncols)],
-                    np.full(ncols * n, 101).astype(dt)))
+        if ncols > 1:
+            a = np.asfortranarray(a)  # (columns of a row-major table: strided)
+        out.append((list(a), np.full(ncols * n, 101).astype(dt)))
     return out
 
 
