@@ -2001,6 +2001,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
         // more cells than kMaxTiles tiles of LDS hold (e.g. 8192 x 8192 count + mean):
         // one pass of global atomics instead, slower but exact
         P.global = true;
+        P.whole = P.tiles_ok = P.run_tiles = P.run_window = false;
         // a finalized mean accumulates its sum and count(v) in the workspace unless the
         // caller asked for those planes too
         P.total = 256;
@@ -2383,9 +2384,10 @@ static int m2_plan(const dsx_points_desc *d, const dsx_view *v, const Plan &P1, 
     d2.window = nullptr;
     d2.reuse_window = 0;
     // (one plane's tiles may fit the tile strategy where the first pass's did not, and the
-    // strategy passed with a stored window is the first pass's)
+    // strategy passed with a stored window is the first pass's; one of global atomics stores
+    // none)
     d2.strategy = P1.run_tiles ? (int32_t)DSX_STRATEGY_WINDOW
-                               : P1.tiles_ok ? d->strategy : (int32_t)DSX_STRATEGY_AUTO;
+                               : P1.tiles_ok || P1.global ? d->strategy : (int32_t)DSX_STRATEGY_AUTO;
     dsx_planes p2;
     memset(&p2, 0, sizeof p2);
     p2.sum = m2;
@@ -2838,12 +2840,13 @@ extern "C" size_t dsx_points_workspace_size(const dsx_points_desc *d, const dsx_
 // The workspace of a call with an m2 plane: its two passes share it.
 static int m2_total(const dsx_points_desc *d, const dsx_view *v, const Plan &P, double *m2, size_t &total) {
     total = P.total;
-    if (P.global || !P.run_window) return DSX_OK;
+    if (!P.global && !P.run_window) return DSX_OK;
     dsx_points_desc d2;
     Plan P2;
     const int st = m2_plan(d, v, P, m2, d2, P2);
     if (st) return st;
-    if (kM2Base + P2.total > total) total = kM2Base + P2.total;
+    const size_t t2 = (P.global ? 0 : kM2Base) + P2.total;
+    if (t2 > total) total = t2;
     return DSX_OK;
 }
 
@@ -2877,18 +2880,28 @@ static int points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_pla
     const Planes out = planes_of(p);
     hipStream_t s = as_stream(stream);
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
+    const bool f32 = d->xy_dtype == DSX_F32;
     if (P.global) {
+        st = f32 ? run_global<float>(d, a, p, out, mean, ws, s) : run_global<double>(d, a, p, out, mean, ws, s);
+        if (st || !m2) return st;
+        // the m2 plane alone may well fit tiles (count, sum, min, max and std of 20M clustered
+        // float32 rows into 4200 x 4000: 8.0 ms a call with global atomics for it too, 5.7 with
+        // a pass of its own), over the same bytes of the workspace
         dsx_planes p2;
         memset(&p2, 0, sizeof p2);
         p2.sum = m2;
-        const bool f32 = d->xy_dtype == DSX_F32;
-        st = f32 ? run_global<float>(d, a, p, out, mean, ws, s) : run_global<double>(d, a, p, out, mean, ws, s);
-        if (st || !m2) return st;
-        return f32 ? run_global<float>(d, a, &p2, planes_of(&p2), p->mean, ws, s)
-                   : run_global<double>(d, a, &p2, planes_of(&p2), p->mean, ws, s);
+        dsx_points_desc d2;
+        Plan P2;
+        if ((st = m2_plan(d, v, P, m2, d2, P2))) return st;
+        const Planes out2 = planes_of(&p2);
+        if (P2.global)
+            return f32 ? run_global<float>(&d2, a, &p2, out2, p->mean, ws, s)
+                       : run_global<double>(&d2, a, &p2, out2, p->mean, ws, s);
+        return f32 ? dispatch_val<float>(&d2, a, P2, out2, p->mean, ws, s, nullptr)
+                   : dispatch_val<double>(&d2, a, P2, out2, p->mean, ws, s, nullptr);
     }
-    if (d->xy_dtype == DSX_F32) return dispatch_val<float>(d, a, P, out, mean, ws, s, m2);
-    return dispatch_val<double>(d, a, P, out, mean, ws, s, m2);
+    return f32 ? dispatch_val<float>(d, a, P, out, mean, ws, s, m2)
+               : dispatch_val<double>(d, a, P, out, mean, ws, s, m2);
 }
 
 extern "C" int dsx_points_agg(const dsx_points_desc *d, const dsx_view *v, const dsx_planes *p,
