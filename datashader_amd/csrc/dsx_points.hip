@@ -41,7 +41,8 @@ static_assert(kStage >= (kFlush - 1) + 64, "a wave's staging holds a partial lin
 constexpr int kPartThreads = 1024;
 constexpr int kTileThreads = 512;
 // largest LDS of one tile workgroup: half of the CU's LDS less a 2 KB margin, so that two
-// tile workgroups always fit on a CU (three when the power-of-two tile takes <= 52 KB).
+// tile workgroups fit on a CU (three when the power-of-two tile takes <= 52 KB); canvases of
+// very many tiles, and the tile strategy where only then its buckets fit, take larger ones.
 // Larger tiles mean fewer tiles, so the scatter writes longer runs per tile.
 constexpr int kTileLds = 78 * 1024;
 constexpr int kMaxTiles = 4096;
@@ -836,8 +837,10 @@ struct PartArgs {
     const uint32_t *seg_count;        // [G * kWaves]
     int64_t seg_cap;
     int32_t ngroups;                  // G (<= kPartThreads)
-    uint32_t tile_cells, tile_shift;  // tile_cells = 1 << tile_shift
+    uint32_t tile_cells, tile_shift;  // tile_cells = 1 << tile_shift (the window strategy's tiles)
     int32_t ntiles;
+    uint32_t btile_cells;             // the tile strategy's tiles, where they are larger
+    int32_t bntiles;
     uint32_t *hist;                   // [G][ntiles]
     unsigned long long *tile_start;   // [ntiles + 1]
     uint32_t *sorted_cell;            // [sink + 64 * G]: the sorted spill, then one
@@ -847,12 +850,19 @@ struct PartArgs {
     // over which tile t's entries are split evenly (*part_len: the largest part size)
     uint32_t *part_start;             // [ntiles + 1]
     uint32_t *part_tile;              // [max_parts] tile of each part
-    int32_t max_parts;
+    int32_t max_parts, bmax_parts;
     uint32_t *part_len;               // [1]
     uint8_t *scratch;                 // one tile-layout region per part of a split tile
     const int32_t *rec;               // the call's window record (its strategy)
     int32_t window_only;              // no tables under the tile strategy (a skipped call)
     uint32_t min_part_tiles;          // fewest blocks a tile part is given (tile strategy)
+
+    // to the tiles of the tile strategy (a kernel of either: if that is the one that runs)
+    __device__ __forceinline__ void take_btiles() {
+        tile_cells = btile_cells;
+        ntiles = bntiles;
+        max_parts = bmax_parts;
+    }
 };
 
 // Block-wide exclusive scan of one value per thread (1024 threads).
@@ -918,9 +928,12 @@ __device__ __forceinline__ uint32_t block_exscan32(uint32_t v, uint32_t *sh, uin
 // place, and the tile total.
 __global__ __launch_bounds__(kPartThreads) void spill_colscan_kernel(PartArgs p,
                                                                     unsigned long long *totals) {
-    if (p.window_only && tiles_run(p.rec)) return;  // uniform
+    const bool tiles = tiles_run(p.rec);
+    if (p.window_only && tiles) return;  // uniform
+    if (tiles) p.take_btiles();
     __shared__ unsigned long long sh[kPartThreads / 64 + 1];
     const int t = blockIdx.x;
+    if (t >= p.ntiles) return;  // uniform
     const int g = threadIdx.x;  // ngroups <= kPartThreads
     const unsigned long long v = g < p.ngroups ? p.hist[(size_t)g * p.ntiles + t] : 0ull;
     unsigned long long tot;
@@ -931,7 +944,9 @@ __global__ __launch_bounds__(kPartThreads) void spill_colscan_kernel(PartArgs p,
 
 __global__ __launch_bounds__(kPartThreads) void spill_tilescan_kernel(PartArgs p,
                                                                      const unsigned long long *totals) {
-    if (p.window_only && tiles_run(p.rec)) return;  // uniform
+    const bool tiles = tiles_run(p.rec);
+    if (p.window_only && tiles) return;  // uniform
+    if (tiles) p.take_btiles();
     __shared__ unsigned long long sh[kPartThreads / 64 + 1];
     unsigned long long carry = 0;
     for (int t0 = 0; t0 < p.ntiles; t0 += blockDim.x) {
@@ -948,7 +963,7 @@ __global__ __launch_bounds__(kPartThreads) void spill_tilescan_kernel(PartArgs p
     // heavier than the mean (the edge of a dense cluster just outside the window) is
     // spread over several workgroups
     // (under the tile strategy the counts are blocks of entries, not entries)
-    const unsigned long long minp = tiles_run(p.rec) ? p.min_part_tiles : (unsigned long long)kMinPart;
+    const unsigned long long minp = tiles ? p.min_part_tiles : (unsigned long long)kMinPart;
     const unsigned long long mean = (carry + p.ntiles - 1) / p.ntiles;
     const unsigned long long e15 = mean + (mean + 1) / 2;
     const unsigned long long E = e15 > minp ? e15 : minp;
@@ -1318,7 +1333,7 @@ __device__ __forceinline__ void fold_parts(uint8_t *smem, const Lay &L, const ui
 // Split tiles: one workgroup per tile folds its parts' scratch regions in LDS and writes
 // the tile.  Tiles of one part were written by tile_agg_kernel.
 template <int KEYB>
-__global__ __launch_bounds__(kTileThreads) void tile_merge_kernel(PartArgs p, Lay L,
+__global__ __launch_bounds__(kTileThreads) void tile_merge_kernel(PartArgs p, Lay Lw, Lay Lb,
                                                                  const int32_t *window, int32_t W,
                                                                  int32_t H, int64_t wcap_px,
                                                                  int32_t ncat, int64_t ncells,
@@ -1326,9 +1341,11 @@ __global__ __launch_bounds__(kTileThreads) void tile_merge_kernel(PartArgs p, La
     extern __shared__ __align__(16) uint8_t smem[];
     const int t = blockIdx.x;
     // only: the strategy whose tiles these are (0: the one that ran)
-    if (t >= p.ntiles || (only == DSX_STRATEGY_TILES && !tiles_run(window)) ||
-        (only == DSX_STRATEGY_WINDOW && tiles_run(window)))
-        return;
+    const bool tiles = tiles_run(window);
+    if ((only == DSX_STRATEGY_TILES && !tiles) || (only == DSX_STRATEGY_WINDOW && tiles)) return;
+    if (tiles) p.take_btiles();
+    const Lay L = tiles ? Lb : Lw;
+    if (t >= p.ntiles) return;
     const uint32_t first = p.part_start[t], nparts = p.part_start[t + 1] - first;
     if (nparts <= 1) return;  // uniform
     fold_parts<kTileThreads, KEYB>(smem, L, p.scratch + (size_t)first * L.bytes, nparts);
@@ -1797,6 +1814,7 @@ __global__ __launch_bounds__(kTileThreads) void btile_agg_kernel(PartArgs p, Bkt
                                                                 int32_t ncat, int64_t ncells,
                                                                 const double *mean, Planes out) {
     if (!tiles_run(window)) return;  // uniform: the window strategy's tile pass runs instead
+    p.take_btiles();
     extern __shared__ __align__(16) uint8_t smem[];
     uint32_t *sblk = reinterpret_cast<uint32_t *>(smem + L.bytes);  // [s.batch]
     // the tile's blocks, in the order of their scan workgroups: workgroup g's run is
@@ -1912,26 +1930,31 @@ __global__ __launch_bounds__(kTileThreads) void btile_agg_kernel(PartArgs p, Bkt
 }
 
 // ---- host side --------------------------------------------------------------------------------
+// A strategy's tiles: runs of 2^shift cells.
+struct Tiles {
+    int shift;
+    int32_t n;
+    int32_t max_parts;   // upper bound of the tile parts (grid of the tile kernel)
+    Lay lay;
+};
+
 struct Plan {
     uint32_t flags;
     int keyb, vbytes;
     Lay wl;              // window layout
-    Lay tl;              // tile layout
+    Tiles wt, bt;        // the window strategy's tiles; the tile strategy's
     int64_t ncells;
-    int32_t ntiles;
     int scan_groups;
     int64_t seg_cap;
-    size_t scan_lds, tile_lds;
+    size_t scan_lds;
     uint32_t o_thist, o_stage_cell, o_stage_val;  // scan LDS offsets
     // workspace offsets
     size_t o_window, o_pad, o_hist_sel, o_count, o_partials, o_spill_cell, o_spill_val, o_hist,
         o_totals, o_tile_start, o_sorted_cell, o_sorted_val, o_part_start, o_part_len, o_part_tile,
         o_scratch, total;
-    int32_t max_parts;   // upper bound of the tile parts (grid of the tile kernel)
     bool whole;          // the window is the whole canvas
     bool global;         // the canvas is too large for the tiles: global-atomic pass
     int bshift, cw, ch;
-    int tshift;          // tile_cells = 1 << tshift
     // the tile strategy (tiles_ok: the tiles' buckets fit the scan's LDS)
     bool tiles_ok;
     bool run_window, run_tiles;  // the strategies this call launches (both under AUTO)
@@ -1981,29 +2004,22 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
         if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
             cus = c;
     }
-    P.tshift = 0;
-    while ((int64_t)(2ll << P.tshift) * cb <= kTileLds - 16) ++P.tshift;
+    const auto tiles_of = [&](int shift) {
+        Tiles t;
+        t.shift = shift;
+        const int64_t n = (P.ncells + (1ll << shift) - 1) >> shift;
+        t.n = (int32_t)(n < 1 ? 1 : n);
+        t.max_parts = 2 * t.n + 1;
+        t.lay = make_lay(P.flags, P.keyb, 1u << shift);
+        return t;
+    };
+    int shift = 0;
+    while ((int64_t)(2ll << shift) * cb <= kTileLds - 16) ++shift;
     // a small canvas still gets one tile per CU (down to 1024-cell tiles): 800x600 counts
     // made 30 tiles of 16384 cells, so 30 workgroups did all of the tile work
-    while (P.tshift > kMinTileShift && ((P.ncells + (1ll << P.tshift) - 1) >> P.tshift) < cus)
-        --P.tshift;
-    while ((P.ncells + (1ll << P.tshift) - 1) >> P.tshift > kMaxTiles) ++P.tshift;
-    // tiles of twice the size (one workgroup a CU) where only their buckets fit the tile
-    // strategy's scan: without it every row of data spread over the canvas is spilled
-    // (count, sum, min, max, std of 20M float64 rows into 1800 x 1000: 847 us a call with
-    // 2048-cell tiles, 434 with 4096).  The strategy asked for has no say: the window's
-    // size follows from the tiles, and a stored window is used again under either.
-    {
-        const size_t vb = (size_t)P.vbytes;
-        const auto fits = [&](int sh) {
-            const size_t nb = (size_t)((P.ncells + (1ll << sh) - 1) >> sh);
-            return bkt_layout(vb, nb, (size_t)kBktMinC, P) <= (size_t)kLdsBytes - 512;
-        };
-        const int64_t ids = 4 * (kBktBatch + 2 * (int64_t)cus + 1);
-        if (!fits(P.tshift) && fits(P.tshift + 1) && (2ll << P.tshift) * cb + 16 + ids <= kLdsBytes)
-            ++P.tshift;
-    }
-    const int64_t tcap = 1ll << P.tshift;
+    while (shift > kMinTileShift && ((P.ncells + (1ll << shift) - 1) >> shift) < cus) --shift;
+    while ((P.ncells + (1ll << shift) - 1) >> shift > kMaxTiles) ++shift;
+    const int64_t tcap = 1ll << shift;
     P.global = false;
     if (tcap * (int64_t)cb > kLdsBytes - 16) {
         // more cells than kMaxTiles tiles of LDS hold (e.g. 8192 x 8192 count + mean):
@@ -2018,17 +2034,30 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
         return DSX_OK;
     }
     if (tcap % kTileThreads) return DSX_ERR_SHAPE;  // never: tiles hold >= 1024 cells
-    P.ntiles = (int32_t)((P.ncells + tcap - 1) >> P.tshift);
-    if (P.ntiles < 1) P.ntiles = 1;
-    P.tl = make_lay(P.flags, P.keyb, (uint32_t)tcap);
-    P.tile_lds = P.tl.bytes;
+    P.wt = P.bt = tiles_of(shift);
+    // The tile strategy takes tiles of twice the size (one workgroup a CU) where only their
+    // buckets fit its scan: without it every row of data spread over the canvas is spilled
+    // (count, sum, min, max, std of 20M float64 rows into 1800 x 1000: 847 us a call with
+    // 2048-cell tiles, 434 with 4096).  The window strategy keeps the small ones (mean of 20M
+    // float32 rows in a hot spot into 3840 x 2160: 288 us a call with large tiles, 268 with
+    // small ones).
+    {
+        const size_t vb = (size_t)P.vbytes;
+        const auto fits = [&](int sh) {
+            const size_t nb = (size_t)((P.ncells + (1ll << sh) - 1) >> sh);
+            return bkt_layout(vb, nb, (size_t)kBktMinC, P) <= (size_t)kLdsBytes - 512;
+        };
+        const int64_t ids = 4 * (kBktBatch + 2 * (int64_t)cus + 1);
+        if (!fits(shift) && fits(shift + 1) && 2 * tcap * cb + 16 + ids <= kLdsBytes)
+            P.bt = tiles_of(shift + 1);
+    }
     // scan LDS: window planes, tile histogram, per-wave spill staging, control words.
     // The window keeps no NaN plane: with count() and count(v) both asked for, rows with
     // a NaN value are spilled and the tile adds them to the window's cells.
     const uint32_t wflags = P.flags & ~PL_NAN;
     const uint32_t cbw = cell_bytes(wflags, P.keyb);
     const size_t stage = (size_t)kWaves * kStage * (4 + (size_t)P.vbytes);
-    const size_t side = align_up((size_t)4 * P.ntiles, 16) + stage + kCtrlBytes;
+    const size_t side = align_up((size_t)4 * P.wt.n, 16) + stage + kCtrlBytes;
     const int64_t wcap_cells = (int64_t)((kLdsBytes - side - 16) / cbw);
     int64_t wcap_px = wcap_cells / ncat;
     if (wcap_px < 1) return DSX_ERR_SHAPE;
@@ -2036,7 +2065,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     if (P.whole) wcap_px = (int64_t)v->width * v->height;
     P.wl = make_lay(wflags, P.keyb, (uint32_t)(wcap_px * ncat));
     P.o_thist = P.wl.bytes;
-    P.o_stage_cell = P.o_thist + (uint32_t)align_up((size_t)4 * P.ntiles, 16);
+    P.o_stage_cell = P.o_thist + (uint32_t)align_up((size_t)4 * P.wt.n, 16);
     P.o_stage_val = P.o_stage_cell + (uint32_t)(kWaves * kStage * 4);
     P.scan_lds = P.wl.bytes + side;
     // coarse selection grid: bins of 2^bshift pixels on a side, at most kSelBins bins
@@ -2059,8 +2088,8 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     P.tiles_ok = false;
     P.batch = kBktBatch;
     // (its scan forms a cell with 24-bit multiplies: py * (W ncat) + px * ncat + category)
-    if (tcap <= (int64_t)kBktMaxTileCells && (int64_t)v->width * ncat < (1ll << 24)) {
-        const size_t vb = (size_t)P.vbytes, nb = (size_t)P.ntiles;
+    if (P.bt.lay.cap <= (uint32_t)kBktMaxTileCells && (int64_t)v->width * ncat < (1ll << 24)) {
+        const size_t vb = (size_t)P.vbytes, nb = (size_t)P.bt.n;
         for (int cs = 8; (1 << cs) >= kBktMinC && !P.tiles_ok; --cs) {
             if ((1 << cs) > kBktMaxC) continue;
             const size_t C = (size_t)1 << cs;
@@ -2081,7 +2110,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
                 // starts its load pipeline over
                 P.batch = kBktBatch;
                 auto blds = [&](size_t nbat) {
-                    return (size_t)P.tl.bytes + 4 * (nbat + 2 * (size_t)P.scan_groups + 1);
+                    return (size_t)P.bt.lay.bytes + 4 * (nbat + 2 * (size_t)P.scan_groups + 1);
                 };
                 while (P.batch < (uint32_t)kBktBatchMax && blds(2 * (size_t)P.batch) <= (size_t)kLdsBytes / 2)
                     P.batch *= 2;
@@ -2102,14 +2131,16 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
     P.o_pad = o; o = align_up(o + kPadBytes, 256);
     P.o_hist_sel = o; o = align_up(o + 4 * (size_t)kSelBins, 256);
     P.o_count = o; o = align_up(o + 4 * (size_t)P.scan_groups * kWaves, 256);  // sub-segment lengths
-    P.o_hist = o; o = align_up(o + 4 * (size_t)P.scan_groups * P.ntiles, 256);
-    P.o_totals = o; o = align_up(o + 8 * (size_t)P.ntiles, 256);
-    P.o_tile_start = o; o = align_up(o + 8 * (size_t)(P.ntiles + 1), 256);
-    P.max_parts = 2 * P.ntiles + 1;
-    P.o_part_start = o; o = align_up(o + 4 * (size_t)(P.ntiles + 1), 256);
+    // (the larger of the two strategies' needs: the window strategy has as many tiles or more)
+    const size_t nt = (size_t)P.wt.n, np = (size_t)P.wt.max_parts;
+    const size_t scratch_w = np * P.wt.lay.bytes, scratch_b = (size_t)P.bt.max_parts * P.bt.lay.bytes;
+    P.o_hist = o; o = align_up(o + 4 * (size_t)P.scan_groups * nt, 256);
+    P.o_totals = o; o = align_up(o + 8 * nt, 256);
+    P.o_tile_start = o; o = align_up(o + 8 * (nt + 1), 256);
+    P.o_part_start = o; o = align_up(o + 4 * (nt + 1), 256);
     P.o_part_len = o; o = align_up(o + 4, 256);
-    P.o_part_tile = o; o = align_up(o + 4 * (size_t)P.max_parts, 256);
-    P.o_scratch = o; o = align_up(o + (size_t)P.max_parts * P.tl.bytes, 256);
+    P.o_part_tile = o; o = align_up(o + 4 * np, 256);
+    P.o_scratch = o; o = align_up(o + (scratch_b > scratch_w ? scratch_b : scratch_w), 256);
     const size_t shared = o;
     P.o_partials = o; o = align_up(o + (size_t)P.scan_groups * P.wl.bytes, 256);
     P.o_spill_cell = o; o = align_up(o + 4 * (nseg + kScatterPad), 256);
@@ -2125,7 +2156,7 @@ static int make_plan(const dsx_points_desc *d, const dsx_view *v, const dsx_plan
         P.o_nblk = o; o = align_up(o + 4 * (size_t)P.scan_groups, 256);
         P.o_bhdr = o; o = align_up(o + 8 * nblocks, 256);
         P.o_bwl = o; o = align_up(o + 4 * nblocks, 256);
-        P.o_blpre = o; o = align_up(o + 4 * (size_t)P.scan_groups * P.ntiles, 256);
+        P.o_blpre = o; o = align_up(o + 4 * (size_t)P.scan_groups * P.bt.n, 256);
         P.o_pool = o; o = align_up(o + (size_t)P.blk_bytes * nblocks, 256);
         end_tiles = o;
     }
@@ -2192,9 +2223,9 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     sa.seg_count = seg_count;
     sa.seg_cap = P.seg_cap;
     sa.hist = reinterpret_cast<uint32_t *>(ws + P.o_hist);
-    sa.tile_cells = P.tl.cap;
-    sa.tile_shift = P.tshift;
-    sa.ntiles = P.ntiles;
+    sa.tile_cells = P.wt.lay.cap;
+    sa.tile_shift = (uint32_t)P.wt.shift;
+    sa.ntiles = P.wt.n;
     sa.o_thist = P.o_thist;
     sa.o_stage_cell = P.o_stage_cell;
     sa.o_stage_val = P.o_stage_val;
@@ -2236,8 +2267,8 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     BktArgs ba;
     if (P.run_tiles) {
         ba.rec = window;
-        ba.nb = P.ntiles;
-        ba.tile_shift = (uint32_t)P.tshift;
+        ba.nb = P.bt.n;
+        ba.tile_shift = (uint32_t)P.bt.shift;
         ba.cshift = P.cshift;
         ba.o_bval = P.o_bval;
         ba.blk_bytes = P.blk_bytes;
@@ -2291,9 +2322,11 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     pa.seg_count = seg_count;
     pa.seg_cap = P.seg_cap;
     pa.ngroups = P.scan_groups;
-    pa.tile_cells = P.tl.cap;
-    pa.tile_shift = P.tshift;
-    pa.ntiles = P.ntiles;
+    pa.tile_cells = P.wt.lay.cap;
+    pa.tile_shift = (uint32_t)P.wt.shift;
+    pa.ntiles = P.wt.n;
+    pa.btile_cells = P.bt.lay.cap;
+    pa.bntiles = P.bt.n;
     pa.hist = reinterpret_cast<uint32_t *>(ws + P.o_hist);
     pa.tile_start = reinterpret_cast<unsigned long long *>(ws + P.o_tile_start);
     pa.sorted_cell = reinterpret_cast<uint32_t *>(ws + P.o_sorted_cell);
@@ -2302,13 +2335,14 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     pa.part_start = reinterpret_cast<uint32_t *>(ws + P.o_part_start);
     pa.part_len = reinterpret_cast<uint32_t *>(ws + P.o_part_len);
     pa.part_tile = reinterpret_cast<uint32_t *>(ws + P.o_part_tile);
-    pa.max_parts = P.max_parts;
+    pa.max_parts = P.wt.max_parts;
+    pa.bmax_parts = P.bt.max_parts;
     pa.scratch = ws + P.o_scratch;
     pa.rec = window;
     pa.window_only = skip ? 1 : 0;
     pa.min_part_tiles = P.tiles_ok ? P.min_part_tiles : (uint32_t)kMinPart;
     unsigned long long *totals = reinterpret_cast<unsigned long long *>(ws + P.o_totals);
-    hipLaunchKernelGGL(spill_colscan_kernel, dim3(P.ntiles), dim3(kPartThreads), 0, st, pa, totals);
+    hipLaunchKernelGGL(spill_colscan_kernel, dim3(P.wt.n), dim3(kPartThreads), 0, st, pa, totals);
     hipLaunchKernelGGL(spill_tilescan_kernel, dim3(1), dim3(kPartThreads), 0, st, pa,
                        (const unsigned long long *)totals);
     if (P.run_window)
@@ -2318,18 +2352,18 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
     if (P.run_window) {
         auto tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV>;
         if constexpr (!SQDEV) {  // the common plane sets: compile-time planes
-            if (P.tl.flags == PL_CNT) tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, PL_CNT>;
-            else if (P.tl.flags == (PL_CNT | PL_SUM))
+            if (P.wt.lay.flags == PL_CNT) tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, PL_CNT>;
+            else if (P.wt.lay.flags == (PL_CNT | PL_SUM))
                 tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, PL_CNT | PL_SUM>;
-            else if (P.tl.flags == (PL_CNTV | PL_SUM))
+            else if (P.wt.lay.flags == (PL_CNTV | PL_SUM))
                 tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, PL_CNTV | PL_SUM>;
-            else if (P.tl.flags == (PL_CNT | PL_SUM | PL_NAN))  // count + mean / sum
+            else if (P.wt.lay.flags == (PL_CNT | PL_SUM | PL_NAN))  // count + mean / sum
                 tile = tile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, PL_CNT | PL_SUM | PL_NAN>;
         }
         e = hipFuncSetAttribute((const void *)tile, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)P.tile_lds);
+                                (int)P.wt.lay.bytes);
         if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-        hipLaunchKernelGGL(tile, dim3(P.max_parts), dim3(kTileThreads), P.tile_lds, st, pa, P.tl,
+        hipLaunchKernelGGL(tile, dim3(P.wt.max_parts), dim3(kTileThreads), P.wt.lay.bytes, st, pa, P.wt.lay,
                            (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, mean, out);
         if ((s = launch_status())) return s;
     }
@@ -2337,33 +2371,34 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
         // (a squared-deviation pass has the sum plane only, one without values the count only)
         constexpr uint32_t kOne = SQDEV ? PL_SUM : HAS_VAL ? 0u : PL_CNT;
         auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV, false, kOne>;
-        if (P.tl.flags != kOne) btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV>;
+        if (P.bt.lay.flags != kOne) btile = btile_agg_kernel<TV, HAS_VAL, KEYB, SQDEV>;
         e = hipFuncSetAttribute((const void *)btile, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)P.btile_lds);
         if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-        hipLaunchKernelGGL(btile, dim3(P.max_parts), dim3(kTileThreads), P.btile_lds, st, pa, ba,
-                           P.tl, (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, mean,
+        hipLaunchKernelGGL(btile, dim3(P.bt.max_parts), dim3(kTileThreads), P.btile_lds, st, pa, ba,
+                           P.bt.lay, (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, mean,
                            out);
         if ((s = launch_status())) return s;
     }
     auto merge = tile_merge_kernel<KEYB>;
+    const size_t merge_lds = P.bt.lay.bytes > P.wt.lay.bytes ? P.bt.lay.bytes : P.wt.lay.bytes;
     e = hipFuncSetAttribute((const void *)merge, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)P.tile_lds);
+                            (int)merge_lds);
     if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-    hipLaunchKernelGGL(merge, dim3(P.ntiles), dim3(kTileThreads), P.tile_lds, st, pa, P.tl,
+    hipLaunchKernelGGL(merge, dim3(P.wt.n), dim3(kTileThreads), merge_lds, st, pa, P.wt.lay, P.bt.lay,
                        (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, out,
                        skip ? (int32_t)DSX_STRATEGY_WINDOW : 0);
     if ((s = launch_status()) || !m2) return s;
     if constexpr (HAS_VAL && !SQDEV) {
         if (P.run_tiles) {  // the same buckets again, one plane (so a smaller region)
-            const Lay L2 = make_lay(PL_SUM, KEYB, P.tl.cap);
+            const Lay L2 = make_lay(PL_SUM, KEYB, P.bt.lay.cap);
             Planes out2;
             memset(&out2, 0, sizeof out2);
             out2.sum = m2;
-            size_t lds = P.btile_lds - P.tl.bytes + L2.bytes;
+            size_t lds = P.btile_lds - P.bt.lay.bytes + L2.bytes;
             auto btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true, false, PL_SUM>;
             // the tile's means in LDS too where two workgroups still fit a CU
-            const size_t o_mean = align_up(lds, 16), with = o_mean + 8 * (size_t)P.tl.cap;
+            const size_t o_mean = align_up(lds, 16), with = o_mean + 8 * (size_t)P.bt.lay.cap;
             if (with <= (size_t)kLdsBytes / 2) {
                 btile = btile_agg_kernel<TV, HAS_VAL, KEYB, true, true, PL_SUM>;
                 ba.o_mean = (uint32_t)o_mean;
@@ -2371,10 +2406,10 @@ static int run_points(const dsx_points_desc *d, const PointArgs &a, const Plan &
             }
             e = hipFuncSetAttribute((const void *)btile, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-            hipLaunchKernelGGL(btile, dim3(P.max_parts), dim3(kTileThreads), lds, st, pa, ba, L2,
+            hipLaunchKernelGGL(btile, dim3(P.bt.max_parts), dim3(kTileThreads), lds, st, pa, ba, L2,
                                (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells,
                                (const double *)out.mean, out2);
-            hipLaunchKernelGGL(merge, dim3(P.ntiles), dim3(kTileThreads), (size_t)L2.bytes, st, pa, L2,
+            hipLaunchKernelGGL(merge, dim3(P.bt.n), dim3(kTileThreads), (size_t)L2.bytes, st, pa, L2, L2,
                                (const int32_t *)window, a.W, a.H, wcap_px, ncat, P.ncells, out2,
                                (int32_t)DSX_STRATEGY_TILES);
             if ((s = launch_status())) return s;
