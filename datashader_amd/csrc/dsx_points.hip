@@ -504,7 +504,8 @@ struct Rows {
 
 // Whether three sets of rows fit the registers of a scan: not the 64-bit category inputs
 // beside float64 coordinates and values (by(int32 codes, mean) over 20M rows, spread over
-// the canvas: 355 us a call with three sets, 307 with two).
+// the canvas: 355 us a call with three sets, 307 with two; by(int32 codes, first), most rows
+// in a hot spot: 282 and 263).
 template <typename TC, typename TV, bool HAS_VAL, int CK>
 constexpr bool kDeepRows = !(CK == CK_ANY && sizeof(TC) == 8 && HAS_VAL && sizeof(TV) == 8);
 
@@ -3063,6 +3064,7 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
     auto *const index = global_ptr(r.index);
     const int64_t nchunks = (a.n + kChunk - 1) / kChunk;
     using R = Rows<TC, TV, true, CK>;
+    constexpr int kAhead = kDeepRows<TC, TV, true, CK> ? 2 : 1;
     auto step = [&](int64_t ck, const R &S, R &far) {
         int64_t cell[kItems];
         bool keep[kItems];
@@ -3081,7 +3083,7 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
         }
 #pragma unroll
         for (int it = 0; it < kItems; ++it) kv[it] = keep[it] ? key[cell[it]] : (typename K::T)0;
-        far.load(a, ck + 2 * (int64_t)gridDim.x, tid);
+        far.load(a, ck + kAhead * (int64_t)gridDim.x, tid);
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             if (!keep[it] || K::key((double)S.v[it]) != kv[it]) continue;
@@ -3092,11 +3094,18 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
     R sa, sb, sc;
     const int64_t G = gridDim.x;
     sa.load(a, blockIdx.x, tid);
-    sb.load(a, blockIdx.x + G, tid);
-    for (int64_t ck = blockIdx.x; ck < nchunks; ck += 3 * G) {  // steps past the end drop rows
-        step(ck, sa, sc);
-        step(ck + G, sb, sa);
-        step(ck + 2 * G, sc, sb);
+    if constexpr (kAhead == 2) {
+        sb.load(a, blockIdx.x + G, tid);
+        for (int64_t ck = blockIdx.x; ck < nchunks; ck += 3 * G) {  // steps past the end drop rows
+            step(ck, sa, sc);
+            step(ck + G, sb, sa);
+            step(ck + 2 * G, sc, sb);
+        }
+    } else {
+        for (int64_t ck = blockIdx.x; ck < nchunks; ck += 2 * G) {
+            step(ck, sa, sb);
+            step(ck + G, sb, sa);
+        }
     }
 }
 
@@ -3243,6 +3252,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     // last chunk reads chunk nchunks (rows past the end: re-reads the last row, dropped)
     auto chunk_of = [&](int64_t k) { return k >= nchunks ? nchunks : (r.last ? nchunks - 1 - k : k); };
     using R = Rows<TC, TV, NANCHK, CK>;
+    constexpr int kAhead = kDeepRows<TC, TV, NANCHK, CK> ? 2 : 1;
     auto *const index = global_ptr(r.index);
     auto *const sindex = global_ptr(reinterpret_cast<long long *>(r.index));
     // Three register sets rotate roles (binned / in flight / being loaded), as in the
@@ -3302,7 +3312,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
             if (thr && out[it]) pth[it] = __hip_atomic_load(index + cell[it] - 1, __ATOMIC_RELAXED,
                                                             __HIP_MEMORY_SCOPE_AGENT);
         }
-        far.load(a, chunk_of(k + 2 * (int64_t)gridDim.x), tid);
+        far.load(a, chunk_of(k + kAhead * (int64_t)gridDim.x), tid);
 #pragma unroll
         for (int it = 0; it < kRiwItems; ++it) {
             if (!out[it]) continue;
@@ -3334,11 +3344,18 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     R sa, sb, sc;
     const int64_t G = gridDim.x;
     sa.load(a, chunk_of(blockIdx.x), tid);
-    sb.load(a, chunk_of(blockIdx.x + G), tid);
-    for (int64_t k = blockIdx.x; k < nchunks; k += 3 * G) {  // steps past the end drop rows
-        step(k, sa, sc);
-        step(k + G, sb, sa);
-        step(k + 2 * G, sc, sb);
+    if constexpr (kAhead == 2) {
+        sb.load(a, chunk_of(blockIdx.x + G), tid);
+        for (int64_t k = blockIdx.x; k < nchunks; k += 3 * G) {  // steps past the end drop rows
+            step(k, sa, sc);
+            step(k + G, sb, sa);
+            step(k + 2 * G, sc, sb);
+        }
+    } else {
+        for (int64_t k = blockIdx.x; k < nchunks; k += 2 * G) {
+            step(k, sa, sb);
+            step(k + G, sb, sa);
+        }
     }
     __syncthreads();
     if constexpr (PK) {

@@ -91,3 +91,32 @@ def test_ends(strategy, kind, ct):
 @pytest.mark.parametrize("ct", [np.float32, np.float64])
 def test_several_chunks_a_workgroup(strategy, kind, n, ct):
     _check(kind, n, ct, 1, np.random.default_rng(n))
+
+
+@pytest.mark.parametrize("n", [5, 8193, 3_200_001])
+@pytest.mark.parametrize("kind", ["codes-int16", "codes-int64", "bin-float64"])
+@pytest.mark.parametrize("ct,vt", [(np.float64, np.float64), (np.float32, np.float64),
+                                   (np.float64, np.float32)])
+def test_selected_rows(kind, n, ct, vt):
+    """The first, the last and the largest value's row of each category (the row-index scans)."""
+    rng = np.random.default_rng(n + 1)
+    x, y = rng.random((2, n)).astype(ct)
+    v = rng.integers(-99, 100, n).astype(vt)  # (ties: the first row is taken)
+    v[::11] = np.nan
+    k, by, cat, ncat = _keys(kind, n, rng)
+    f = dsa.DeviceFrame({c: _column(a, 1) for c, a in (("x", x), ("y", y), ("v", v), ("k", k))},
+                        categories={"k": list("abcd")} if by == "k" else None)
+    cvs = dsa.Canvas(W, H, x_range=XR, y_range=YR)
+    b = cf.point_bins(x, y, G.view_for(W, H, XR, YR), W, H)
+    ok = np.flatnonzero((b >= 0) & (cat >= 0) & ~np.isnan(v))
+    cell = b[ok] * ncat + cat[ok]
+    first, last, top = (np.full(W * H * ncat, -1, np.int64) for _ in range(3))
+    first[cell[::-1]] = ok[::-1]
+    last[cell] = ok
+    order = np.lexsort((ok, -v[ok]))[::-1]
+    top[cell[order]] = ok[order]
+    for red, want in ((dsa.first("v"), first), (dsa.last("v"), last)):
+        exp = np.where(want < 0, np.nan, v[want].astype(np.float64)).reshape(H, W, ncat)
+        np.testing.assert_array_equal(cvs.points(f, "x", "y", dsa.by(by, red)).values, exp)
+    got = cvs.points(f, "x", "y", dsa.by(by, dsa.where(dsa.max("v")))).values
+    np.testing.assert_array_equal(got, top.reshape(H, W, ncat))
