@@ -104,6 +104,7 @@ def upload(blocks):
     host = area.numpy()
     work = pieces(blocks)
     flat = [t.view(-1) for _, t in blocks]
+    stream = torch.cuda.current_stream(flat[0].device)
     jobs, done = [], []
 
     def stage(i):
@@ -120,7 +121,7 @@ def upload(blocks):
                 dst = flat[b][first:first + k]
                 dst.copy_(area[at:at + k * dst.element_size()].view(dst.dtype), non_blocking=True)
             ev = torch.cuda.Event()
-            ev.record(torch.cuda.current_stream(flat[0].device))
+            ev.record(stream)
             done.append(ev)
             # (two pieces' DMA stay queued while the one before them gives its memory back)
             if i >= 2 and i - 2 + PIECES < len(work):
@@ -132,6 +133,5 @@ def upload(blocks):
         for f in jobs:
             if not f.cancelled():
                 f.exception()
-        for ev in done[-PIECES:]:
-            ev.synchronize()
+        stream.synchronize()  # (not the last event: a piece that failed half-way has none)
         _give(area)
