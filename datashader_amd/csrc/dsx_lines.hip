@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a, Planes p) {
 // result never depends on the box.  Random LDS u32 atomics run at 5.1 T/s here, global
 // ones at 14-27 G/s.
 constexpr int kBoxThreads = 1024;
-constexpr int kBoxLds = 160 * 1024 - 1024;  // the box, less 1 KB for the kernels' own words
+constexpr int kBoxLds = 160 * 1024 - 1024;  // a run's box, less 1 KB for the kernel's own words
 
 // The box's counters in the workgroup's dynamic LDS.
 extern __shared__ uint32_t box_cells[];
@@ -360,16 +360,14 @@ __device__ __forceinline__ void box_flush(const Box &b, uint32_t *count, int32_t
 // projected once (not once per segment it ends), in 32 bits, and only segments that
 // clipping could shorten take draw_segment: telling those by an inexact float32 delta sent
 // a lane of nearly every wave there (values near zero), 2.21 against 1.54 ms.  The
-// fixed-point walk, its common steps without a lane mask: 1.54 -> 1.12 ms.  Before all of
+// fixed-point walk, its common steps without a lane mask: 1.54 -> 1.13 ms.  Before all of
 // it 2.89 ms (2048 x 1024).
 constexpr int kStripMaxK = 8;        // segments per strip
+// The band alone takes the LDS; what the lanes share is in scalar registers.  (A few words of
+// it in LDS cost the band two columns at some heights, whose pixels then take global atomics:
+// 0.7M x 32 series into 1812 x 803, segments wider than the band, 9.9 ms against 8.2.)
+constexpr int kStripLds = 160 * 1024;
 
-struct StripSeg {
-    int32_t px0, px1;  // snapped ends
-    int32_t flags;     // SEG_* bits
-    int32_t pad;
-    double x0, x1;
-};
 enum : int32_t {
     SEG_FAST = 1,   // both ends in the view and in the band's columns, unclipped in x
     SEG_SKIP = 2,   // nothing of it can be drawn (an end missing, or both outside)
@@ -396,8 +394,6 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
                                                                          int32_t k,
                                                                          int32_t pitch,
                                                                          int64_t lpb) {
-    // (after the band in dynamic LDS: with no static LDS the band starts at address 0)
-    StripSeg *s_seg = reinterpret_cast<StripSeg *>(box_cells + ((a.H * pitch + 3) & ~3));
     const TX *X = reinterpret_cast<const TX *>(a.x);
     const int64_t nseg = a.nverts - 1;
     const int64_t j0 = (int64_t)blockIdx.x * k;
@@ -423,27 +419,38 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
     put.box.cols = pitch; put.box.rows = a.H; put.box.pitch = pitch;
     for (int i = tid; i < a.H * pitch; i += kBoxThreads) box_cells[i] = 0u;
     const int32_t xxmax = snap_max(a.xxmax), yymax = snap_max(a.yymax);
-    if (tid <= ns) {  // (one past the last: read ahead, never drawn)
-        const int64_t j = j0 + (tid < ns ? tid : ns - 1);
-        const TX x0c = X[j * a.xvs], x1c = X[(j + 1) * a.xvs];
+    // Lane q of every wave works out vertex q's column in the band and segment q's flags;
+    // then they are uniform values (16 bits a column: those of a segment outside the band are
+    // not read).
+    uint64_t cols_a, cols_b;  // vertices 0-3, 4-7
+    uint32_t col_c, flags_all = 0u;
+    {
+        const int q = tid & 63, q0 = q < ns ? q : ns, q1 = q + 1 < ns ? q + 1 : ns;
+        const TX x0c = X[(j0 + q0) * a.xvs], x1c = X[(j0 + q1) * a.xvs];
+        const TX xp = X[(j0 + q0 > 0 ? j0 + q0 - 1 : 0) * a.xvs];
         const double x0 = (double)x0c, x1 = (double)x1c;
-        StripSeg g;
-        g.x0 = x0; g.x1 = x1; g.pad = 0; g.flags = 0;
-        g.px0 = snap_in<LOG>(x0, a.sx, a.tx, xxmax, a.xlog);
-        g.px1 = snap_in<LOG>(x1, a.sx, a.tx, xxmax, a.xlog);
-        const auto col = [&](int32_t c) {
+        const int32_t px0 = snap_in<LOG>(x0, a.sx, a.tx, xxmax, a.xlog);
+        const int32_t px1 = snap_in<LOG>(x1, a.sx, a.tx, xxmax, a.xlog);
+        const auto in_band = [&](int32_t c) {
             return c >= 0 && c < a.W && (uint32_t)(c - put.box.c0) < (uint32_t)pitch;
         };
-        if (a.xmin <= x0 && x0 <= a.xmax && a.xmin <= x1 && x1 <= a.xmax && col(g.px0) &&
-            col(g.px1) && unclipped(x0, (double)(TX)(x1c - x0c), a.xmin, a.xmax))
-            g.flags |= SEG_FAST;
+        int32_t f = 0;
+        if (a.xmin <= x0 && x0 <= a.xmax && a.xmin <= x1 && x1 <= a.xmax && in_band(px0) &&
+            in_band(px1) && unclipped(x0, (double)(TX)(x1c - x0c), a.xmin, a.xmax))
+            f |= SEG_FAST;
         if (x0 != x0 || x1 != x1 || (x0 < a.xmin && x1 < a.xmin) || (x0 > a.xmax && x1 > a.xmax))
-            g.flags |= SEG_SKIP;
-        if (j > 0) {
-            const TX xp = X[(j - 1) * a.xvs];
-            if (xp != xp) g.flags |= SEG_START;
-        }
-        s_seg[tid] = g;
+            f |= SEG_SKIP;
+        if (j0 + q0 > 0 && xp != xp) f |= SEG_START;
+        const int32_t c = (px0 - put.box.c0) & 0xFFFF;
+        uint32_t cl[9];
+#pragma unroll
+        for (int i = 0; i <= kStripMaxK; ++i) cl[i] = (uint32_t)__builtin_amdgcn_readlane(c, i);
+#pragma unroll
+        for (int i = 0; i < kStripMaxK; ++i)
+            flags_all |= (uint32_t)__builtin_amdgcn_readlane(f, i) << (4 * i);
+        cols_a = (uint64_t)(cl[0] | cl[1] << 16) | (uint64_t)(cl[2] | cl[3] << 16) << 32;
+        cols_b = (uint64_t)(cl[4] | cl[5] << 16) | (uint64_t)(cl[6] | cl[7] << 16) << 32;
+        col_c = cl[8];
     }
     __syncthreads();
     const uint32_t pitch4 = (uint32_t)pitch * 4u;
@@ -459,15 +466,18 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
         bool in0 = a.ymin <= y0 && y0 <= a.ymax;
         // (a log10 of nothing in the view is not worked out)
         int32_t py0 = !LOG || in0 ? snap_in<LOG>(y0, a.sy, a.ty, yymax, a.ylog) : -1;
-        int4 g = *reinterpret_cast<const int4 *>(&s_seg[0]);  // px0, px1, flags
+        uint64_t ca = cols_a, cb = cols_b;
+        uint32_t cc = col_c, fl = flags_all;
         // segments drawn from the front of a shifting register window (a rolled loop with
         // constant register indices: one copy of the rasteriser, no indexed registers)
 #pragma unroll 1
         for (int q = 0; q < ns; ++q) {
-            const int32_t px0 = __builtin_amdgcn_readfirstlane(g.x);
-            const int32_t px1 = __builtin_amdgcn_readfirstlane(g.y);
-            const int32_t flags = __builtin_amdgcn_readfirstlane(g.z);
-            g = *reinterpret_cast<const int4 *>(&s_seg[q + 1]);
+            const int32_t px0 = put.box.c0 + (int32_t)(ca & 0xFFFFu), flags = (int32_t)(fl & 15u);
+            ca = ca >> 16 | cb << 48;
+            cb = cb >> 16 | (uint64_t)cc << 48;
+            cc = 0u;
+            fl >>= 4;
+            const int32_t px1 = put.box.c0 + (int32_t)(ca & 0xFFFFu);
             const TY y0c = row.y[0], y1c = row.y[1];
             const double y1 = (double)y1c;
             const bool in1 = a.ymin <= y1 && y1 <= a.ymax;
@@ -492,8 +502,8 @@ __global__ __launch_bounds__(kBoxThreads) void lines_xconst_strip_kernel(LineArg
                     // (both ends beyond one bound, or one missing: nothing is drawn)
                     const bool none = y0 != y0 || y1 != y1 || (y0 < a.ymin && y1 < a.ymin) ||
                                       (y0 > a.ymax && y1 > a.ymax);
-                    if (!none && segment_ends<TX, TY>(a, start, (TX)s_seg[q].x0, (TX)s_seg[q].x1,
-                                                      y0c, y1c, e)) {
+                    if (!none && segment_ends<TX, TY>(a, start, X[(j0 + q) * a.xvs],
+                                                      X[(j0 + q + 1) * a.xvs], y0c, y1c, e)) {
                         draw = put.box.has(e.x0, e.y0) && put.box.has(e.x1, e.y1) && e.x0 < a.W &&
                                e.x1 < a.W;
                         if (!draw) put.walk<int32_t>(e.start, e.x0, e.x1, e.y0, e.y1, e.clipped);
@@ -675,7 +685,7 @@ static int cu_count() {
 template <typename TX, typename TY>
 static int launch_strips(const LineArgs &a, uint32_t *count, int64_t nstrips, int64_t nblocks,
                          int64_t k, int64_t pitch, int64_t lpb, hipStream_t s) {
-    const size_t lds = (size_t)4 * ((a.H * pitch + 3) & ~3) + sizeof(StripSeg) * (kStripMaxK + 1);
+    const size_t lds = (size_t)4 * a.H * pitch;
     // (two band sizes, so that few registers hold samples a strip does not have)
     auto kern = k <= 4 ? lines_xconst_strip_kernel<TX, TY, 4, false>
                        : lines_xconst_strip_kernel<TX, TY, kStripMaxK, false>;
@@ -764,7 +774,7 @@ extern "C" int dsx_lines_agg(const dsx_lines_desc *d, const dsx_view *v, const d
     hipStream_t s = as_stream(stream);
     const bool x32 = d->x_dtype == DSX_F32, y32 = d->y_dtype == DSX_F32;
     // x-constant series with count / any only: LDS strips
-    int64_t pitch = kBoxLds / (4 * (int64_t)v->height);
+    int64_t pitch = kStripLds / (4 * (int64_t)v->height);
     if (pitch % 2 == 0) --pitch;
     const bool counts = !d->val && d->cat.kind == DSX_CAT_NONE && acc->count && !needs_val;
     if (counts && d->axis == 1 && d->x_line_stride == 0 && pitch >= 5) {

@@ -22,6 +22,8 @@ import datashader_amd as dsa  # noqa: E402
     (2, 700, 1000),     # one segment a line, wider than the fixed-point steps
     (17, 200, 255),     # no walk beyond them
     (17, 200, 257),     # a step or two beyond
+    (9, 30, 8192),      # the band takes all of the LDS
+    (32, 1812, 803),    # segments wider than the band
     (300, 1900, 1080)])
 def test_mixed_walks(nverts, W, H, values, dtype):
     rng = np.random.default_rng(nverts + H)
