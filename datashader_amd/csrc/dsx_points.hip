@@ -26,8 +26,6 @@
 #include <math.h>
 #include <string.h>
 
-#include <type_traits>
-
 #include "dsx_project.h"
 
 namespace dsx {
@@ -504,10 +502,83 @@ struct Rows {
     __device__ __forceinline__ uint32_t code8(int it) const { return (c8[it / kPer] >> (8 * (it % kPer))) & 0xFFu; }
 };
 
+// The rows of a chunk as the row-index passes read them: a thread's rows lie a workgroup apart
+// (row it * kScanThreads + tid), one load a row and column; WIDE (float32 columns on 16-byte
+// boundaries, a row count divisible by four, no category): four consecutive ones, one 16-byte
+// load a column.  The grouped loads of Rows lose here although they bring the rows faster: the
+// first chunks' rows then read their cells before the other workgroups' atomics have landed,
+// and more of them take an atomic of their own (first, window pass, 2.1M float32 rows into 250 x
+// 400: 141 us so, 161 with Rows; 2.1M float64 rows 62 and 74; at 12M rows Rows gains 2 to 5 %
+// with first, nothing with where).
+// A row past the end re-reads the last one and is dropped when binned.
+template <typename TC, typename TV, bool HAS_VAL, int CK, bool WIDE = false>
+struct SpreadRows {
+    static_assert(!WIDE || (sizeof(TC) == 4 && (!HAS_VAL || sizeof(TV) == 4) && CK == CK_NONE && kItems == 4),
+                  "wide rows: float32 columns, four rows a thread");
+    TC x[kItems], y[kItems];
+    TV v[kItems];
+    int64_t c[kItems];  // CK_ANY: the raw categorizer inputs; CK_CODE8: the bytes
+
+    __device__ __forceinline__ void load(const PointArgs &a, int64_t ck, int tid) {
+        int64_t b = ck * kChunk;
+        if constexpr (WIDE) {
+            typedef float Vec __attribute__((ext_vector_type(4)));
+            uint32_t lastq;  // the last readable group of four rows
+            if (b >= a.n) {  // a prefetch past the end: re-read the last four rows
+                b = a.n - 4;
+                lastq = 0;
+            } else {
+                const int64_t rem = a.n - b;
+                lastq = rem >= kChunk ? (uint32_t)(kChunk / 4 - 1) : (uint32_t)(rem / 4 - 1);
+            }
+            const uint32_t q = (uint32_t)tid < lastq ? (uint32_t)tid : lastq;
+            const Vec vx = stream_load(reinterpret_cast<const Vec *>(reinterpret_cast<const float *>(a.x) + b) + q);
+            const Vec vy = stream_load(reinterpret_cast<const Vec *>(reinterpret_cast<const float *>(a.y) + b) + q);
+            Vec vv = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (HAS_VAL)
+                vv = stream_load(reinterpret_cast<const Vec *>(reinterpret_cast<const float *>(a.val) + b) + q);
+#pragma unroll
+            for (int it = 0; it < kItems; ++it) {
+                x[it] = vx[it];
+                y[it] = vy[it];
+                v[it] = (TV)vv[it];
+                c[it] = 0;
+            }
+            return;
+        }
+        uint32_t lastj;  // the last readable row of the chunk
+        if (b >= a.n) {
+            b = a.n > 0 ? a.n - 1 : 0;
+            lastj = 0;
+        } else {
+            const int64_t rem = a.n - b;
+            lastj = rem >= kChunk ? (uint32_t)(kChunk - 1) : (uint32_t)(rem - 1);
+        }
+        const TC *X = reinterpret_cast<const TC *>(a.x) + b, *Y = reinterpret_cast<const TC *>(a.y) + b;
+        const TV *V = reinterpret_cast<const TV *>(a.val) + (HAS_VAL ? b : 0);
+#pragma unroll
+        for (int it = 0; it < kItems; ++it) {
+            uint32_t j = (uint32_t)(it * kScanThreads + tid);
+            j = j < lastj ? j : lastj;
+            x[it] = stream_load(X + j);
+            y[it] = stream_load(Y + j);
+            if constexpr (HAS_VAL) v[it] = stream_load(V + j);
+            else v[it] = TV(0);
+            if constexpr (CK == CK_CODE8) c[it] = reinterpret_cast<const uint8_t *>(a.cat.col)[b + j];
+            else if constexpr (CK == CK_ANY) c[it] = load_cat_raw(a.cat, b + j);
+            else c[it] = 0;
+        }
+    }
+    // row `it`'s place in the chunk
+    static __device__ __forceinline__ int32_t place(int it, int tid) {
+        return WIDE ? 4 * tid + it : it * kScanThreads + tid;
+    }
+    __device__ __forceinline__ uint32_t code8(int it) const { return (uint32_t)c[it]; }
+};
+
 // Whether three sets of rows fit the registers of a scan: not the 64-bit category inputs
 // beside float64 coordinates and values (by(int32 codes, mean) over 20M rows, spread over
-// the canvas: 355 us a call with three sets, 307 with two; by(int32 codes, first), most rows
-// in a hot spot: 282 and 263).
+// the canvas: 355 us a call with three sets, 307 with two).
 template <typename TC, typename TV, bool HAS_VAL, int CK>
 constexpr bool kDeepRows = !(CK == CK_ANY && sizeof(TC) == 8 && HAS_VAL && sizeof(TV) == 8);
 
@@ -583,14 +654,14 @@ __device__ __forceinline__ int32_t scan_category(const Cat &c, const R &rows, in
     return (int32_t)category_raw(c, rows.c[it]);
 }
 
-// Pixel of a loaded row, false when it is dropped.  LIN: locate_xy without branches, for a
+// Pixel of a loaded row, false when it is dropped (own: it is the thread's).  LIN: locate_xy without branches, for a
 // view whose translation is exactly -xmin*sx, -ymin*sy (lin_view): an in-range row then
 // projects into [0, W] -- x >= xmin gives fl(x*sx) >= fl(xmin*sx) -- so the wraparound and
 // the lower bound never apply; a row out of range (NaN included) converts to anything
 // (cvt_sat_i32) and is dropped.
 template <bool LIN, typename R>
-__device__ __forceinline__ bool scan_pixel(const PointArgs &a, const R &rows, int it, int32_t &px,
-                                           int32_t &py) {
+__device__ __forceinline__ bool scan_pixel(const PointArgs &a, const R &rows, int it, bool own,
+                                           int32_t &px, int32_t &py) {
     if constexpr (LIN) {
         const double x = (double)rows.x[it], y = (double)rows.y[it];
         const bool inr = (a.xmin <= x) & (x <= a.xmax) & (a.ymin <= y) & (y <= a.ymax);
@@ -598,10 +669,10 @@ __device__ __forceinline__ bool scan_pixel(const PointArgs &a, const R &rows, in
         const int32_t yy = cvt_sat_i32(__dadd_rn(__dmul_rn(y, a.sy), a.ty));
         px = xx < a.W - 1 ? xx : a.W - 1;
         py = yy < a.H - 1 ? yy : a.H - 1;
-        return rows.own(it) & inr;
+        return own & inr;
     } else {
         px = py = 0;
-        return rows.own(it) && locate_xy(a, rows.x[it], rows.y[it], px, py);
+        return own && locate_xy(a, rows.x[it], rows.y[it], px, py);
     }
 }
 
@@ -649,7 +720,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(PointArgs a, ScanArg
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             int32_t px, py, pc = 0;
-            bool keep = scan_pixel<LIN>(a, cur, it, px, py);
+            bool keep = scan_pixel<LIN>(a, cur, it, cur.own(it), px, py);
             if constexpr (CK != CK_NONE) {
                 pc = scan_category<CK>(a.cat, cur, it);
                 keep = keep && pc >= 0;
@@ -1634,7 +1705,7 @@ __global__ __launch_bounds__(kScanThreads) void bscan_kernel(PointArgs a, BktArg
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             int32_t px, py, pc = 0;
-            bool keep = scan_pixel<LIN>(a, cur, it, px, py);
+            bool keep = scan_pixel<LIN>(a, cur, it, cur.own(it), px, py);
             if constexpr (CK == CK_CODE8) {
                 const uint32_t b8 = cur.code8(it);
                 const uint32_t k = b8 - (b8 >= c8_at ? c8_sub : 0u);
@@ -3065,16 +3136,17 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
     const auto *const key = global_ptr(reinterpret_cast<const typename K::T *>(r.key));
     auto *const index = global_ptr(r.index);
     const int64_t nchunks = (a.n + kChunk - 1) / kChunk;
-    using R = Rows<TC, TV, true, CK>;
-    constexpr int kAhead = kDeepRows<TC, TV, true, CK> ? 2 : 1;
+    using R = SpreadRows<TC, TV, true, CK>;
     auto step = [&](int64_t ck, const R &S, R &far) {
+        const int64_t rem64 = a.n - ck * kChunk;  // rows of this chunk, uniform
+        const int32_t rem = rem64 >= kChunk ? kChunk : (rem64 > 0 ? (int32_t)rem64 : 0);
         int64_t cell[kItems];
         bool keep[kItems];
         typename K::T kv[kItems];
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             int32_t px, py, pc = 0;
-            bool k_ = scan_pixel<LIN>(a, S, it, px, py);
+            bool k_ = scan_pixel<LIN>(a, S, it, S.place(it, tid) < rem, px, py);
             if constexpr (CK != CK_NONE) {
                 pc = scan_category<CK>(a.cat, S, it);
                 k_ = k_ && pc >= 0;
@@ -3085,7 +3157,7 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
         }
 #pragma unroll
         for (int it = 0; it < kItems; ++it) kv[it] = keep[it] ? key[cell[it]] : (typename K::T)0;
-        far.load(a, ck + kAhead * (int64_t)gridDim.x, tid);
+        far.load(a, ck + 2 * (int64_t)gridDim.x, tid);
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             if (!keep[it] || K::key((double)S.v[it]) != kv[it]) continue;
@@ -3096,25 +3168,18 @@ __global__ __launch_bounds__(kScanThreads) void rowindex_arg_kernel(RiArgs r) {
     R sa, sb, sc;
     const int64_t G = gridDim.x;
     sa.load(a, blockIdx.x, tid);
-    if constexpr (kAhead == 2) {
-        sb.load(a, blockIdx.x + G, tid);
-        for (int64_t ck = blockIdx.x; ck < nchunks; ck += 3 * G) {  // steps past the end drop rows
-            step(ck, sa, sc);
-            step(ck + G, sb, sa);
-            step(ck + 2 * G, sc, sb);
-        }
-    } else {
-        for (int64_t ck = blockIdx.x; ck < nchunks; ck += 2 * G) {
-            step(ck, sa, sb);
-            step(ck + G, sb, sa);
-        }
+    sb.load(a, blockIdx.x + G, tid);
+    for (int64_t ck = blockIdx.x; ck < nchunks; ck += 3 * G) {  // steps past the end drop rows
+        step(ck, sa, sc);
+        step(ck + G, sb, sa);
+        step(ck + 2 * G, sc, sb);
     }
 }
 
 template <typename TC>
 static int rowindex_launch(const RiArgs &r, int val_dtype, hipStream_t st) {
     const bool arg = r.mode == DSX_RI_ARGMAX || r.mode == DSX_RI_ARGMIN;
-    if (arg && r.a.n >= 4) {  // the streaming form
+    if (arg) {  // the streaming form
         const PointArgs &a = r.a;
         const bool lin = lin_view(a), byte = cat_kind(a.cat) == CK_CODE8;
         const int64_t chunks = (a.n + kChunk - 1) / kChunk;
@@ -3180,7 +3245,7 @@ struct RiwArgs {
 struct RiwPlan {
     uint32_t cap;
     int groups, bshift, cw, ch;
-    size_t lds, o_window, o_pad, o_hist, o_partials, total;
+    size_t lds, o_window, o_hist, o_partials, total;
 };
 
 static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, bool packed = false,
@@ -3207,7 +3272,6 @@ static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, boo
     P.ch = (v->height + (1 << P.bshift) - 1) >> P.bshift;
     size_t o = 0;
     P.o_window = o; o = align_up(o + 4 * kRecWords, 256);
-    P.o_pad = o; o = align_up(o + kPadBytes, 256);
     P.o_hist = o; o = align_up(o + 4 * (size_t)kSelBins, 256);
     P.o_partials = o; o = align_up(o + cb * (size_t)P.cap * (size_t)P.groups, 256);
     P.total = o;
@@ -3216,8 +3280,8 @@ static int riw_plan(const dsx_points_desc *d, const dsx_view *v, RiwPlan &P, boo
 
 // NANCHK: rows whose value is NaN are skipped (the value column is read); CK, LIN: as
 // in scan_kernel (the category read with the row's other columns, the branch-free linear
-// projection); PK: the packed ARGMAX / ARGMIN form (float32 values).
-template <typename TC, typename TV, bool NANCHK, int CK, bool LIN, bool PK = false>
+// projection); PK: the packed ARGMAX / ARGMIN form (float32 values); WIDE: as in SpreadRows.
+template <typename TC, typename TV, bool NANCHK, int CK, bool LIN, bool PK = false, bool WIDE = false>
 __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r) {
     static_assert(kRiwThreads == kScanThreads && kRiwItems == kItems, "chunks as the scan's");
     static_assert(!PK || sizeof(TV) == 4, "packed: float32 values");
@@ -3253,8 +3317,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     // that after the first sweep most rows fail the global skip test; a step past the
     // last chunk reads chunk nchunks (rows past the end: re-reads the last row, dropped)
     auto chunk_of = [&](int64_t k) { return k >= nchunks ? nchunks : (r.last ? nchunks - 1 - k : k); };
-    using R = Rows<TC, TV, NANCHK, CK>;
-    constexpr int kAhead = kDeepRows<TC, TV, NANCHK, CK> ? 2 : 1;
+    using R = SpreadRows<TC, TV, NANCHK, CK, WIDE>;
     auto *const index = global_ptr(r.index);
     auto *const sindex = global_ptr(reinterpret_cast<long long *>(r.index));
     // Three register sets rotate roles (binned / in flight / being loaded), as in the
@@ -3262,10 +3325,12 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     // device-scope load, served by L2) before any atomic: most rows cannot improve the
     // cell.  Those reads are issued before the loads of the chunk two ahead and waited for
     // after them, so that wait (vector memory counts complete in order) does not also wait
-    // for those loads.  more: whether the step loads a set.
-    auto step = [&](int64_t k, const R &S, R &far, auto more) {
+    // for those loads.
+    auto step = [&](int64_t k, const R &S, R &far) {
         const int64_t ck = chunk_of(k);
         const int64_t row0 = ck * kChunk;
+        const int64_t rem64 = a.n - row0;  // rows of this chunk, uniform
+        const int32_t rem = rem64 >= kChunk ? kChunk : (rem64 > 0 ? (int32_t)rem64 : 0);
         int64_t cell[kRiwItems];
         long long cur[kRiwItems];
         unsigned long long pkv[kRiwItems];  // PK: the row's packed value
@@ -3274,7 +3339,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
 #pragma unroll
         for (int it = 0; it < kRiwItems; ++it) {
             int32_t px, py, pc = 0;
-            bool keep = scan_pixel<LIN>(a, S, it, px, py);
+            bool keep = scan_pixel<LIN>(a, S, it, S.place(it, tid) < rem, px, py);
             if constexpr (CK != CK_NONE) {
                 pc = scan_category<CK>(a.cat, S, it);
                 keep = keep && pc >= 0;
@@ -3314,7 +3379,7 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
             if (thr && out[it]) pth[it] = __hip_atomic_load(index + cell[it] - 1, __ATOMIC_RELAXED,
                                                             __HIP_MEMORY_SCOPE_AGENT);
         }
-        if constexpr (decltype(more)::value) far.load(a, chunk_of(k + kAhead * (int64_t)gridDim.x), tid);
+        far.load(a, chunk_of(k + 2 * (int64_t)gridDim.x), tid);
 #pragma unroll
         for (int it = 0; it < kRiwItems; ++it) {
             if (!out[it]) continue;
@@ -3346,24 +3411,11 @@ __global__ __launch_bounds__(kRiwThreads) void rowindex_window_kernel(RiwArgs r)
     R sa, sb, sc;
     const int64_t G = gridDim.x;
     sa.load(a, chunk_of(blockIdx.x), tid);
-    if constexpr (kAhead == 2) {
-        sb.load(a, chunk_of(blockIdx.x + G), tid);
-        // (the last steps by themselves: carried through the loop they load and bin rows past
-        // the end, up to five chunks of them a workgroup -- first over 5M float64 rows spread
-        // over 300 x 200: 87 us with them, 76 without)
-        int64_t k = blockIdx.x;
-        for (; k + 2 * G < nchunks; k += 3 * G) {
-            step(k, sa, sc, std::true_type());
-            step(k + G, sb, sa, std::true_type());
-            step(k + 2 * G, sc, sb, std::true_type());
-        }
-        if (k < nchunks) step(k, sa, sc, std::false_type());
-        if (k + G < nchunks) step(k + G, sb, sc, std::false_type());
-    } else {
-        for (int64_t k = blockIdx.x; k < nchunks; k += 2 * G) {
-            step(k, sa, sb, std::true_type());
-            step(k + G, sb, sa, std::true_type());
-        }
+    sb.load(a, chunk_of(blockIdx.x + G), tid);
+    for (int64_t k = blockIdx.x; k < nchunks; k += 3 * G) {  // steps past the end drop rows
+        step(k, sa, sc);
+        step(k + G, sb, sa);
+        step(k + 2 * G, sc, sb);
     }
     __syncthreads();
     if constexpr (PK) {
@@ -3500,12 +3552,23 @@ static int riw_launch(const dsx_points_desc *d, const RiwArgs &r, const RiwPlan 
         else if (byte) kern = rowindex_window_kernel<TC, float, false, CK_CODE8, false, true>;
         else kern = rowindex_window_kernel<TC, float, false, CK_ANY, false, true>;
     }
+    if constexpr (sizeof(TC) == 4) {
+        const bool wide = lin && a.cat.kind == DSX_CAT_NONE && d->n >= 4 && d->n % 4 == 0 &&
+                          ((uintptr_t)a.x % 16) == 0 && ((uintptr_t)a.y % 16) == 0 &&
+                          (!nan || (f32v && ((uintptr_t)a.val % 16) == 0));
+        if (wide) {
+            if (r.packed)
+                kern = nan ? rowindex_window_kernel<TC, float, true, CK_NONE, true, true, true>
+                           : rowindex_window_kernel<TC, float, false, CK_NONE, true, true, true>;
+            else
+                kern = nan ? rowindex_window_kernel<TC, float, true, CK_NONE, true, false, true>
+                           : rowindex_window_kernel<TC, double, false, CK_NONE, true, false, true>;
+        }
+    }
     const hipError_t e = hipFuncSetAttribute((const void *)kern,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
     if (e != hipSuccess) { record_hip_error(e); return DSX_ERR_HIP; }
-    RiwArgs rk = r;
-    rk.a = pad_rows(r.a, sizeof(TC) == 8, nan ? (f32v ? 4 : 8) : 0, ws + P.o_pad, st);
-    hipLaunchKernelGGL(kern, dim3(P.groups), dim3(kRiwThreads), P.lds, st, rk);
+    hipLaunchKernelGGL(kern, dim3(P.groups), dim3(kRiwThreads), P.lds, st, r);
     if ((s = launch_status())) return s;
     hipLaunchKernelGGL(rowindex_window_merge, dim3(grid_for(P.cap, 256, 4)), dim3(256), 0, st, r,
                        P.groups);
