@@ -650,7 +650,11 @@ __global__ __launch_bounds__(kBoxThreads) void lines_run_kernel(LineArgs a, uint
                 box_flush(put.box, count, a.W, a.H);
                 __syncthreads();
             }
-            put.box = place_box(bx0, bx1, by0, by1, a.W, a.H, cap);
+            // (the last round's box is no larger than its bounds: cleared and added whole, one of
+            // the LDS's size costs some 5 us, for a track of 100k vertices a third of the kernel)
+            const int32_t bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;
+            put.box = fits && base + kRunSegs >= s1 ? Box{bx0, by0, bw, bh, bw | 1}
+                                                    : place_box(bx0, bx1, by0, by1, a.W, a.H, cap);
             for (int i = tid; i < put.box.rows * put.box.pitch; i += kBoxThreads) box_cells[i] = 0u;
             __syncthreads();
         }
@@ -794,12 +798,16 @@ extern "C" int dsx_lines_agg(const dsx_lines_desc *d, const dsx_view *v, const d
                               : launch_strips<double, double>(a, p.count, nstrips, nblocks, k, pitch, lpb, s));
         }
     }
-    // axis 0 with count / any only: runs of segments through an LDS box, from the size where
-    // it beats one global atomic a pixel (calls on 1900 x 1000: 10k segments 75 against 68 us,
-    // 20k 60 against 68, 100k 60 against 67-96, 10M 0.25 against 6.1 ms); lines shorter than
-    // a workgroup would each clear and add a box for few segments
+    // axis 0 with count / any only: runs of segments through an LDS box, from the size where the
+    // middle of a time series is drawn sooner so than by a global atomic a pixel (kernels, 762 x
+    // 426: 20k vertices 12.8 against 16.6 us, 30k 17.6 against 14.9, 100k 26.7 against 15.9; all
+    // of the series 30k 13.0 against 9.2, 200k 58 against 10; 10M into 900 x 525 6.1 against
+    // 0.24 ms a call).  A smooth track has few pixels a segment and stays with the atomics' time
+    // longer (100k vertices 8.5 against 9.0 us, the middle of it 6.0 against 11.4), which the host
+    // part of a call hides.  Lines shorter than a workgroup would each clear and add a box for
+    // few segments.
     if (counts && d->axis == 0 && d->nverts > kBoxThreads && d->nlines <= 65535 &&
-        d->nlines * (d->nverts - 1) >= 16384)
+        d->nlines * (d->nverts - 1) >= 32768)
         return x32 ? (y32 ? launch_runs<float, float>(a, p.count, s) : launch_runs<float, double>(a, p.count, s))
                    : (y32 ? launch_runs<double, float>(a, p.count, s) : launch_runs<double, double>(a, p.count, s));
     const int block = 256;

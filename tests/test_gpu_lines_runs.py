@@ -35,7 +35,7 @@ def _lines(xs, ys, W, H, xr, yr):
     return got, exp
 
 
-@pytest.mark.parametrize("m,n", [(3, 9001), (257, 4097), (300, 6145), (520, 4099)])
+@pytest.mark.parametrize("m,n", [(3, 10_924), (7, 9001), (257, 4097), (300, 6145), (520, 4099)])
 def test_lines_split_into_runs(m, n):
     rng = np.random.default_rng(m)
     xs, ys = np.cumsum(rng.normal(0, 1, (2, m, n)), axis=2).astype(np.float32)
@@ -58,6 +58,24 @@ def _blocks(kind, n, rng):
     out = (what == 5)[:, None] & (rng.random((m, 4096)) < 0.99)
     x[out] = np.nan
     return x.reshape(-1)[:n], y.reshape(-1)[:n]
+
+
+@pytest.mark.parametrize("n", [32_768, 32_769, 32_770, 65_535])
+@pytest.mark.parametrize("W,H", [(1900, 1000), (640, 1), (1, 480), (30_000, 4)])
+def test_first_sizes(W, H, n):
+    """The smallest lines drawn in runs (boxes no larger than a round's pixels), in full and with
+    a view in the middle."""
+    rng = np.random.default_rng(n)
+    t = np.arange(n, dtype=np.float64)
+    noisy = np.cumsum(rng.normal(0, 1, n)) + rng.normal(0, 9, n)
+    track = np.cumsum(rng.normal(0, 1, (2, n)), axis=1)
+    track[0][::97] = np.nan
+    for x, y in ((t, noisy), (track[0], track[1])):
+        for cut in (0.0, 0.25):
+            xr, yr = ((float(np.nanquantile(a, cut)), float(np.nanquantile(a, 1 - cut))) for a in (x, y))
+            got, exp = _lines(x[None], y[None], W, H, xr, yr)
+            assert exp.sum() > 0
+            np.testing.assert_array_equal(got, exp)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
@@ -108,11 +126,11 @@ def test_axes_and_types(xd, yd, xt, yt):
         np.testing.assert_array_equal(got, exp)
 
 
-@pytest.mark.parametrize("chunk_rows", [16_384, 20_000, 33_333])
+@pytest.mark.parametrize("chunk_rows", [32_766, 32_769, 50_001])
 def test_streamed_chunks(chunk_rows):
     """A line in chunks long enough for the runs: the vertices before a chunk are context, and a
     partition's first chunk goes on from the last partition's row without drawing it again."""
-    n = 101_003
+    n = 160_003
     rng = np.random.default_rng(chunk_rows)
     x, y = np.cumsum(rng.normal(0, 0.05, (2, n)), axis=1)
     for at in range(0, n, chunk_rows):  # (gaps at, before and after the chunks' first rows)
@@ -127,7 +145,7 @@ def test_streamed_chunks(chunk_rows):
     np.testing.assert_array_equal(resident.values, oracle.line_axis0(x, y, view, W, H)["count"])
     streamed = cvs.line(dsa.ChunkedFrame(df, chunk_rows=chunk_rows), "x", "y", agg=dsa.count())
     np.testing.assert_array_equal(streamed.values, resident.values)
-    cuts = [0, 40_000, 62_000, n]
+    cuts = [0, 70_000, 105_000, n]
     parts = [df.iloc[a:b] for a, b in zip(cuts[:-1], cuts[1:])]
     got = cvs.line(dsa.ChunkedFrame(parts, chunk_rows=chunk_rows), "x", "y", agg=dsa.count())
     want = np.zeros((H, W), np.int64)
