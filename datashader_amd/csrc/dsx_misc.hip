@@ -64,9 +64,10 @@ __device__ __forceinline__ void minmax_reduce_block(double &lo, double &hi, doub
 // Each thread reads pieces of kPiece consecutive rows (16 bytes, one load; the rows before
 // the first 16-byte boundary and after the last whole piece go to one thread each), a grid
 // stride apart, kBoundsU of them a step, and the next step's loads are issued before this
-// one's rows are compared; a piece past the end re-reads the last one, so the last step
-// is no serial tail.  HBM bound: 20M float64 rows 37 us (one 8-byte load a row, the rows of
-// the last step one by one) -> 31; 10M 17 -> 15; the column streams past the caches (read once).
+// one's rows are compared; a piece past the end re-reads the step's first one (all threads at
+// one line cost 3M float32 rows 7 of 37 us), and a thread past it loads no step more.  HBM
+// bound: 20M float64 rows 37 us (one 8-byte load a row, the rows of the last step one by one)
+// -> 31; 10M 17 -> 15; the column streams past the caches (read once).
 constexpr int kBoundsU = 4;
 
 template <typename T>
@@ -97,7 +98,7 @@ __global__ __launch_bounds__(kBoundsBlock) void bounds_partial(const T *a, int64
 #pragma unroll
             for (int u = 0; u < kBoundsU; ++u) {
                 const int64_t j = i + u * stride;
-                v[u] = __builtin_nontemporal_load(p + (j < np ? j : np - 1));
+                v[u] = __builtin_nontemporal_load(p + (j < np ? j : i));
             }
         };
         auto fold = [&](const Vec (&v)[kBoundsU]) {
@@ -107,10 +108,12 @@ __global__ __launch_bounds__(kBoundsBlock) void bounds_partial(const T *a, int64
                 for (int e = 0; e < kPiece; ++e) take(v[u][e]);
         };
         load(x, t);
-        for (int64_t i = t; i < np; i += 2 * kBoundsU * stride) {
-            load(y, i + kBoundsU * stride);
+        for (int64_t i = t + kBoundsU * stride;; i += 2 * kBoundsU * stride) {
+            if (i >= np) { fold(x); break; }
+            load(y, i);
             fold(x);
-            load(x, i + 2 * kBoundsU * stride);
+            if (i + kBoundsU * stride >= np) { fold(y); break; }
+            load(x, i + kBoundsU * stride);
             fold(y);
         }
     }
